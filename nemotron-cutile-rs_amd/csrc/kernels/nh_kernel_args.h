@@ -220,6 +220,15 @@ struct GemmW8A8Args {
     int32_t pad_;
 };
 
+// G3 with both operands loaded straight into registers (gemm_direct.hip).
+struct GemmDirectArgs {
+    GemmW8A8Args g;     // xq: tiled A; wq: tiled int8 [N][K], or tiled INT4 (then sw is unused)
+    int32_t groups;     // row groups: group q owns M tiles [q T / groups, (q + 1) T / groups), T = ceil(M / 16)
+    int32_t w4_zp;      // INT4: zero point
+    float w4_scale;     // and tensor scale
+    int32_t pad_;
+};
+
 // R1: sigmoid top-k routing, one wave per token.
 struct RouteArgs {
     const float* scores;  // [T][E]

@@ -6,3 +6,4 @@
 #include "gemm_f32.hip"
 #include "moe.hip"
 #include "gemm_persistent.hip"
+#include "gemm_direct.hip"

@@ -216,6 +216,100 @@ bool use_persistent_224(const nh_context* ctx, const void* xq, const float* sx, 
     return tiles_p >= cu && work_p < work_o;
 }
 
+// The LDS-tiled G3 kernels (gemm.hip) on tiled A, largest first.
+struct GemmCfg {
+    KernelId id;
+    int bm, bn, threads;
+    size_t lds;  // ring of stages + the tile's scales and bias
+};
+
+const GemmCfg kTiledCfgs[] = {{K_GEMM_TA_256, 256, 128, 1024, gemm_lds_bytes(256, 128, 3)},
+                              {K_GEMM_TA_128, 128, 128, 512, gemm_lds_bytes(128, 128, 3)},
+                              {K_GEMM_TA_64, 64, 128, 384, gemm_lds_bytes(64, 128, 3)},
+                              {K_GEMM_TA_6464, 64, 64, 384, gemm_lds_bytes(64, 64, 3)}};
+
+int64_t gemm_tiles(const GemmCfg& c, int M, int N) {
+    return (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+}
+
+// The largest whose tiles fill every CU, else 64 x 64 (the most tiles); null
+// when the LDS holds none.
+const GemmCfg* tiled_gemm_cfg(const nh_context* ctx, int M, int N) {
+    for (const GemmCfg& c : kTiledCfgs)
+        if (gemm_tiles(c, M, N) >= ctx->cu_count && c.lds <= ctx->max_shared_per_block) return &c;
+    return kTiledCfgs[3].lds <= ctx->max_shared_per_block ? &kTiledCfgs[3] : nullptr;
+}
+
+// The time of that choice in us (cold weights; fitted with plan_direct): a
+// launch and, per round of workgroups and 64-deep K tile, what the kernel's
+// stage loop takes whatever the tile holds.
+double tiled_gemm_us(const nh_context* ctx, int M, int N, int kt) {
+    static const double launch_us[] = {5.0, 4.5, 3.5, 3.0}, kt_us[] = {0.467, 0.292, 0.255, 0.217},
+                        fill[] = {1.0, 0.9, 0.85, 0.8};
+    const GemmCfg* c = tiled_gemm_cfg(ctx, M, N);
+    if (!c) return 1e30;
+    const int at = (int)(c - kTiledCfgs);
+    return launch_us[at] + kt_us[at] * kt * std::max(1.0, fill[at] * (double)gemm_tiles(*c, M, N) / ctx->cu_count);
+}
+
+// The register-direct GEMM (gemm_direct.hip): its tile for a shape, and the
+// time its launch takes, in us.
+struct DirectPlan {
+    KernelId id;
+    int nr, groups;
+    unsigned grid;
+    double us;
+};
+
+// Fitted to 216 shapes of 17..512 rows, 1024..16384 columns and K = 1024..8192
+// (cold weights): a launch, then per round of workgroups an epilogue, and
+// per K tile the fragments through the CU's load path (66 KiB per us), or the
+// weights from HBM (5.6 TB/s) where that is longer.  Against the LDS tiles
+// (tiled_gemm_us), both sides measured at M x N x K: 17 x 2688 x 2688 5.5 / 11.8
+// us, 77 x 6144 x 4096 11.5 / 15.8, 400 x 2688 x 4096 15.5 / 20.9, 64 x 16384 x
+// 1024 7.8 / 6.8, 512 x 16384 x 4096 49.2 / 36.2.
+DirectPlan plan_direct(const nh_context* ctx, int M, int N, int kt, bool w4) {
+    DirectPlan best{};
+    best.us = 1e30;
+    const int mtiles = (M + 15) / 16;
+    const double cu = ctx->cu_count;
+    for (int nr : {1, 2, 4, 8}) {
+        if (nr == 8 && !w4) break;
+        const int maxr = nr == 8 ? 4 : 8;
+        const int groups = (mtiles + maxr - 1) / maxr;
+        const int mr = (mtiles + groups - 1) / groups;
+        const int64_t tn = (N + 16 * nr - 1) / (16 * nr), wgs = tn * groups;
+        if ((tn + 7) / 8 * 8 * groups > kMaxGrid) continue;
+        const double rounds = std::max(1.0, 1.15 * (double)wgs / cu);
+        const double load = rounds * kt * (mr + (w4 ? 0.5 : 1.0) * nr) / 66.0;
+        const double hbm = (double)N * kt * (w4 ? 32 : 64) / 5.6e6;
+        const double us = 2.2 + rounds * (1.2 + 0.07 * mr * nr) + std::max(load, hbm);
+        if (us >= best.us) continue;
+        const KernelId id8[] = {K_GEMM_DIRECT16, K_GEMM_DIRECT32, K_GEMM_DIRECT64, K_GEMM_DIRECT64};
+        const KernelId id4[] = {K_GEMM_W4_DIRECT16, K_GEMM_W4_DIRECT32, K_GEMM_W4_DIRECT64, K_GEMM_W4_DIRECT128};
+        const int at = nr == 1 ? 0 : nr == 2 ? 1 : nr == 4 ? 2 : 3;
+        best = DirectPlan{w4 ? id4[at] : id8[at], nr, groups, (unsigned)((tn + 7) / 8 * 8 * groups), us};
+    }
+    return best;
+}
+
+// What W4A8 takes through the expanded form: a pass that reads the INT4 tiles
+// and writes int8 ones (4096 -> 16384: 17.6 us, 5.7 TB/s), then the int8 product.
+double w4_expanded_us(const nh_context* ctx, size_t m, size_t n, size_t k) {
+    const int kt = (int)tiled_k_tiles(k);
+    const double expand = 2.0 + (double)n * kt * 96 / 5.7e6;
+    return expand + std::min(tiled_gemm_us(ctx, (int)m, (int)n, kt), plan_direct(ctx, (int)m, (int)n, kt, false).us);
+}
+
+nh_status launch_gemm_direct(nh_context* ctx, const DirectPlan& p, const GemmW8A8Args& g, int w4_zp, float w4_scale,
+                             nh_stream stream, nh_error* err) {
+    GemmDirectArgs d{g, p.groups, w4_zp, w4_scale, 0};
+    d.g.tiles_n = (g.N + 16 * p.nr - 1) / (16 * p.nr);
+    // partial fragments of 4 waves, row and column scales, bias, INT4 row sums
+    const size_t lds = 4 * 16 * 1024 + 3 * 128 * 4 + 4 * 128 * 4;
+    return launch(ctx, p.id, p.grid, 256u, lds, stream, d, err);
+}
+
 // G3 launch.  a_tiled: xq holds A in the weights' tiled layout (written by
 // the row quantizer with 16 rows per tile), else row-major [M][K].
 nh_status launch_gemm(nh_context* ctx, const int8_t* xq, const float* sx, const int8_t* wq, const float* sw,
@@ -242,28 +336,19 @@ nh_status launch_gemm(nh_context* ctx, const int8_t* xq, const float* sx, const 
         const unsigned grid = (unsigned)std::min<int64_t>(tiles, ctx->cu_count);
         return launch(ctx, K_GEMM_P224, grid, 512u, kP224Lds, stream, a, err);
     }
-    // Tile choice.  Tiled A: the largest of 256x128 (8 compute + 8 loader
-    // waves), 128x128, 64x128 and 64x64 whose tiles fill every CU, else
-    // 64x64 (the most tiles): M = 128 at 4096 -> 16384 took 34.4 us on 128
-    // workgroups of 256x128 and 28.5 on 256 of 64x128; M = 256 41.0 -> 35.0 on
-    // 128x128.  Row-major A: 256x128 unless that leaves most CUs idle, then
-    // 128x128.
-    struct Cfg {
-        KernelId id;
-        int bm, bn, threads;
-        size_t lds;  // ring of stages + the tile's scales and bias
-    };
-    const Cfg big = {a_tiled ? K_GEMM_TA_256 : K_GEMM_W8A8, 256, 128, 1024, gemm_lds_bytes(256, 128, 3)};
-    const Cfg small = a_tiled ? Cfg{K_GEMM_TA_128, 128, 128, 512, gemm_lds_bytes(128, 128, 3)}
-                              : Cfg{K_GEMM_W8A8_128, 128, 128, 256, gemm_lds_bytes(128, 128, 3)};
-    auto tiles = [&](const Cfg& c) { return (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn); };
-    const Cfg tiny = {K_GEMM_TA_64, 64, 128, 384, gemm_lds_bytes(64, 128, 3)};
-    const Cfg tiny2 = {K_GEMM_TA_6464, 64, 64, 384, gemm_lds_bytes(64, 64, 3)};
-    const Cfg* cfg = nullptr;
+    // Tile choice, tiled A (tiled_gemm_cfg): M = 128 at 4096 -> 16384 took
+    // 34.4 us on 128 workgroups of 256x128 and 28.5 on 256 of 64x128; M = 256
+    // 41.0 -> 35.0 on 128x128.  Row-major A: 256x128 unless that leaves most
+    // CUs idle, then 128x128.
+    const GemmCfg big = a_tiled ? kTiledCfgs[0] : GemmCfg{K_GEMM_W8A8, 256, 128, 1024, gemm_lds_bytes(256, 128, 3)};
+    const GemmCfg small = a_tiled ? kTiledCfgs[1] : GemmCfg{K_GEMM_W8A8_128, 128, 128, 256, gemm_lds_bytes(128, 128, 3)};
+    auto tiles = [&](const GemmCfg& c) { return gemm_tiles(c, M, N); };
+    const GemmCfg* cfg = nullptr;
     if (a_tiled) {
-        for (const Cfg* c : {&big, &small, &tiny, &tiny2})
-            if (!cfg && tiles(*c) >= ctx->cu_count && c->lds <= ctx->max_shared_per_block) cfg = c;
-        if (!cfg && tiny2.lds <= ctx->max_shared_per_block) cfg = &tiny2;
+        cfg = tiled_gemm_cfg(ctx, M, N);
+        // the register-direct kernel where it is faster: few or ragged tiles, long K
+        const DirectPlan p = plan_direct(ctx, M, N, a.kt, false);
+        if (p.us < tiled_gemm_us(ctx, M, N, a.kt)) return launch_gemm_direct(ctx, p, a, 0, 0.0f, stream, err);
     } else if (tiles(big) >= ctx->cu_count / 4 && big.lds <= ctx->max_shared_per_block) {
         cfg = &big;
     } else if (small.lds <= ctx->max_shared_per_block) {
@@ -290,7 +375,7 @@ nh_status launch_gemm(nh_context* ctx, const int8_t* xq, const float* sx, const 
     // half a round instead of 6.
     const int64_t cu = ctx->cu_count;
     const int64_t nbig = (int64_t)a.tiles_m * a.tiles_n;
-    if (cfg == &big && small.lds <= ctx->max_shared_per_block && nbig > cu && nbig % cu != 0 &&
+    if (cfg->id == big.id && small.lds <= ctx->max_shared_per_block && nbig > cu && nbig % cu != 0 &&
         nbig % cu <= cu / 2) {
         const int tn_main = (int)(nbig / cu * cu / a.tiles_m);  // N tiles of whole rounds
         const int n_main = tn_main * big.bn;
@@ -431,6 +516,22 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
         float* sw = (float*)(w8 + align256((size_t)tiled_bytes(n, k)));
         void* lin = (char*)sw + align256(n * sizeof(float));
         const size_t lin_bytes = workspace_bytes - (size_t)((char*)lin - (char*)workspace);
+        // up to a few hundred rows: the register-direct GEMM on the INT4 tiles
+        // themselves.  Its A tiles take the place of the expanded weights
+        // (the linear workspace where there are more rows than columns).
+        const DirectPlan p = plan_direct(ctx, (int)m, (int)n, (int)tiled_k_tiles(k), true);
+        const size_t at_bytes = (size_t)tiled_bytes(m, k);
+        const bool in_w8 = at_bytes <= (size_t)tiled_bytes(n, k);
+        if ((in_w8 || m > kTiledActRows) && p.us < w4_expanded_us(ctx, m, n, k)) {
+            int8_t* atiles = in_w8 ? w8 : (int8_t*)lin;
+            float* sx = in_w8 ? (float*)lin : (float*)((char*)lin + align256(at_bytes));
+            if ((st = launch_quantize(ctx, x, x_dtype, m, k, nullptr, sx, nullptr, atiles, stream, err, 16, nullptr, 1,
+                                      nonfinite, kStageInput)))
+                return st;
+            GemmW8A8Args g{atiles, sx, (const int8_t*)w4_tiled, nullptr, bias, out, (int)m, (int)n, (int)k, 0, 0,
+                           out_dtype, 0, (int)tiled_k_tiles(k), (int)n, 0};
+            return launch_gemm_direct(ctx, p, g, (int)zero_point, scale, stream, err);
+        }
         ExpandInt4Args e{w4_tiled, w8, sw, (int64_t)(tiled_int4_bytes(n, k) / 8), (int64_t)n, scale,
                          (int32_t)zero_point};
         if ((st = launch(ctx, K_EXPAND_INT4, grid_for(e.lanes, 256), 256, 0, stream, e, err))) return st;

@@ -64,6 +64,13 @@ const char* const kKernelSymbols[K_COUNT] = {  // in KernelId order
     "nh_gemm_f32_mfma_bf16_kernel",      // K_GEMM_F32_MFMA_BF16
     "nh_gemm_f32_mfma_any_kernel",       // K_GEMM_F32_MFMA_ANY
     "nh_quantize_rows_r11_kernel",       // K_QUANTIZE_ROWS_R11
+    "nh_gemm_w8a8_direct16_kernel",      // K_GEMM_DIRECT16
+    "nh_gemm_w8a8_direct32_kernel",      // K_GEMM_DIRECT32
+    "nh_gemm_w8a8_direct64_kernel",      // K_GEMM_DIRECT64
+    "nh_gemm_w4a8_direct16_kernel",      // K_GEMM_W4_DIRECT16
+    "nh_gemm_w4a8_direct32_kernel",      // K_GEMM_W4_DIRECT32
+    "nh_gemm_w4a8_direct64_kernel",      // K_GEMM_W4_DIRECT64
+    "nh_gemm_w4a8_direct128_kernel",     // K_GEMM_W4_DIRECT128
 };
 
 void clear_error(nh_error* err) {

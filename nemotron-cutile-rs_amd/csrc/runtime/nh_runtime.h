@@ -67,6 +67,13 @@ enum KernelId : int {
     K_GEMM_F32_MFMA_BF16,     // ... bf16 lhs
     K_GEMM_F32_MFMA_ANY,      // ... any alignment, K and N
     K_QUANTIZE_ROWS_R11,      // row quantizer, 256 threads per row, up to 2816 chunks in registers
+    K_GEMM_DIRECT16,          // G3 straight from registers, up to 128 rows x 16 columns per workgroup
+    K_GEMM_DIRECT32,          // x 32
+    K_GEMM_DIRECT64,          // x 64
+    K_GEMM_W4_DIRECT16,       // the same on tiled INT4 weights
+    K_GEMM_W4_DIRECT32,
+    K_GEMM_W4_DIRECT64,
+    K_GEMM_W4_DIRECT128,      // up to 64 rows x 128 columns
     K_COUNT
 };
 
