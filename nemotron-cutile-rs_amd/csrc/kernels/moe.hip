@@ -444,8 +444,9 @@ extern "C" __global__ __launch_bounds__(512) void nh_moe_grouped_gemm_kernel(Gro
     }
 }
 
-// R3 for the MoE layer (A in slot order).  One workgroup per (expert, half
-// of its N tiles): the chip runs one of them per CU in a single round.  The
+// R3 for the MoE layer (A in slot order).  One workgroup per (expert with
+// routes, part of its N tiles), as many parts as give every CU one workgroup:
+// the chip runs them in a single round.  The
 // expert's routed rows are staged once per pass of up to 16 * row_blocks
 // slots into LDS as 1 KiB MFMA A tiles (direct-to-LDS loads, lane l fetching
 // row l % 16, bytes 16 (l / 16) of its 64-byte K tile, so the fragment reads
@@ -574,16 +575,41 @@ __device__ __forceinline__ void expert_stream(const ExpertGemmArgs& a, v4i (&b0)
     }
 }
 
+// The n-th expert (from 0) whose segment of offsets is not empty, and that
+// segment; -1 when fewer have routes.  Workgroups are dealt to the XCDs and
+// their shader engines in strict rotation, so the experts with routes go to
+// consecutive workgroups: with one workgroup slot per expert, some engines got
+// two rounds of work and others none (16 tokens over 128 experts in 3 parts
+// each: 82 us per projection against 60 in 2 parts).
+__device__ __forceinline__ int nth_active_expert(const int32_t* offsets, int E, int n, int lane, int& seg0, int& seg1) {
+    for (int base = 0; base < E; base += 64) {
+        const int e = min(base + lane, E - 1);
+        const int lo = offsets[e], hi = base + lane < E ? offsets[e + 1] : lo;
+        const uint64_t live = __ballot(hi > lo);
+        const int c = __popcll(live);
+        if (n < c) {
+            const uint64_t below = live & ((1ull << lane) - 1ull);
+            const uint64_t hit = __ballot(((live >> lane) & 1) != 0 && __popcll(below) == n);
+            const int l = __ffsll((unsigned long long)hit) - 1;
+            seg0 = __builtin_amdgcn_readlane(lo, l);
+            seg1 = __builtin_amdgcn_readlane(hi, l);
+            return base + l;
+        }
+        n -= c;
+    }
+    return -1;
+}
+
 // The three forms of the expert-block kernel:
 //  kExpertPlain  A codes in slot order (aq, sa) staged by direct-to-LDS loads;
 //  kExpertOmax   the same, and each workgroup also writes, for every row of
 //                its segment, the largest finite |out| over its own columns
-//                (omax[row][blockIdx.x], f32 bits) and reports non-finite
+//                (omax[row][part], f32 bits) and reports non-finite
 //                outputs: the up projection of the MoE layer, whose output
 //                the down projection requantizes per row;
 //  kExpertQuantA A rows in f32 (ah), quantized per row while staged, with
-//                the row scale RN(amax / 127) from amax = the larger of the
-//                row's two omax entries: the max of the finite |h| over the
+//                the row scale RN(amax / 127) from amax = the largest of the
+//                row's omax entries: the max of the finite |h| over the
 //                whole row, so the codes and scales are those of
 //                nh_quantize_rows_i8 on h (the down projection; K <= 2048:
 //                a wave stages 4 K tiles of each row block).  That fuses
@@ -591,10 +617,18 @@ __device__ __forceinline__ void expert_stream(const ExpertGemmArgs& a, v4i (&b0)
 //                two projections instead of a launch and an int8 copy.
 template <int MODE>
 __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds) {
-    const int e = blockIdx.y;
-    const int seg0 = a.offsets[e], seg1 = a.offsets[e + 1];
-    if (seg0 >= seg1) return;  // no routes: the expert's weights are never read
+    // workgroup b: part b % parts of the (b / parts)-th expert (compact: that has routes)
     const int lane = threadIdx.x & 63;
+    const int part = (int)blockIdx.x % a.parts;
+    int e = (int)blockIdx.x / a.parts, seg0, seg1;
+    if (a.compact) {
+        e = nth_active_expert(a.offsets, a.experts, e, lane, seg0, seg1);
+        if (e < 0) return;  // fewer experts have routes
+    } else {
+        seg0 = a.offsets[e];
+        seg1 = a.offsets[e + 1];
+        if (seg0 >= seg1) return;  // no routes: the expert's weights are never read
+    }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int NW = a.streams;
     const int r16 = lane & 15, g = lane >> 4;
@@ -602,11 +636,11 @@ __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds
     const int nch = (kt + kExpertSlab - 1) / kExpertSlab;
     const int RB = a.row_blocks, cap = 16 * RB;
     const int ntiles = (N + 15) / 16;
-    const int t_begin = blockIdx.x * a.tiles_per_wg;
+    const int t_begin = part * a.tiles_per_wg;
     const int t_end = min(t_begin + a.tiles_per_wg, ntiles);
     if (t_begin >= t_end) {  // uniform: no columns here, so no output of this range is non-zero
         if constexpr (MODE == kExpertOmax)
-            for (int row = seg0 + (int)threadIdx.x; row < seg1; row += blockDim.x) a.omax[row * 2 + blockIdx.x] = 0u;
+            for (int row = seg0 + (int)threadIdx.x; row < seg1; row += blockDim.x) a.omax[(int64_t)row * a.parts + part] = 0u;
         return;
     }
     const int my_tiles = t_begin + wave < t_end ? (t_end - t_begin - wave + NW - 1) / NW : 0;
@@ -709,14 +743,22 @@ __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds
             //    two-deep pipeline of 4 K tiles per lane, with this wave's
             //    first two weight chunks issued behind the first two blocks
             const __amdgpu_buffer_rsrc_t hr = make_rsrc(a.ah, (uint32_t)a.a_rows * (uint32_t)K * 4u);
-            uint32_t hm[4][2];
+            // the rows' maxima over the parts that wrote them, two parts per
+            // round trip (non-negative floats order like their bits)
+            uint32_t hm[4] = {0, 0, 0, 0};
             __builtin_amdgcn_sched_barrier(0);
+            for (int p = 0; p < a.ah_parts; p += 2) {
+                uint32_t h0[4], h1[4];
 #pragma unroll
-            for (int rb = 0; rb < 4; ++rb) {
-                const int row = p0 + rb * 16 + r16;
-                const bool ok = rb < nrb && row < seg1;
-                hm[rb][0] = ok ? a.ahmax[row * 2] : 0u;
-                hm[rb][1] = ok ? a.ahmax[row * 2 + 1] : 0u;
+                for (int rb = 0; rb < 4; ++rb) {
+                    const int row = p0 + rb * 16 + r16;
+                    const bool ok = rb < nrb && row < seg1;
+                    const uint32_t* at = a.ahmax + (int64_t)row * a.ah_parts + p;
+                    h0[rb] = ok ? at[0] : 0u;
+                    h1[rb] = ok && p + 1 < a.ah_parts ? at[1] : 0u;
+                }
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb) hm[rb] = max(hm[rb], max(h0[rb], h1[rb]));
             }
             v4i hv[2][4][4];
             // the lane's 16 values of a K tile: 64 contiguous bytes in either order
@@ -738,7 +780,7 @@ __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds
             };
             auto consume = [&](int rb, const v4i (&buf)[4][4]) {
                 if (rb >= nrb) return;  // uniform
-                const float sc = scale_from_amax(fmaxf(f32_from_bits(hm[rb][0]), f32_from_bits(hm[rb][1])));
+                const float sc = scale_from_amax(f32_from_bits(hm[rb]));
                 const float rcp = sc > 0.0f ? 1.0f / sc : 0.0f;
                 const bool pow2 = scale_is_pow2(sc);
                 if (g == 0) sas[rb * 16 + r16] = sc;
@@ -788,7 +830,7 @@ __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds
         lds_publish();  // the pass's A and scale reads are done before the next pass restages them
         if constexpr (MODE == kExpertOmax)
             if ((int)threadIdx.x < nrb * 16 && p0 + (int)threadIdx.x < seg1)
-                a.omax[(p0 + threadIdx.x) * 2 + blockIdx.x] = lmax[threadIdx.x];
+                a.omax[(int64_t)(p0 + threadIdx.x) * a.parts + part] = lmax[threadIdx.x];
     }
 }
 

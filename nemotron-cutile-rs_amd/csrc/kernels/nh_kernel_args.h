@@ -295,15 +295,15 @@ struct ExpertGemmArgs {
     float* out;              // [R][N]
     int32_t N, K, kt;
     int32_t a_rows;          // R
-    int32_t waves;           // unused (1)
+    int32_t parts;           // workgroups per expert, each owning tiles_per_wg N tiles
     int32_t streams;         // waves per workgroup, each streaming its own N tiles
     int32_t tiles_per_wg;
     int32_t relu2;
     int32_t row_blocks;      // 16-row blocks of A staged per pass (1..4)
     // fused forms of the MoE layer (null when unused):
-    uint32_t* omax;          // [R][2] per workgroup column range: max finite |out| of each row (f32 bits)
+    uint32_t* omax;          // [R][parts] per workgroup column range: max finite |out| of each row (f32 bits)
     const float* ah;         // [R][K] f32 A rows, quantized per row while staged (aq unused)
-    const uint32_t* ahmax;   // [R][2] the omax of the launch that wrote ah
+    const uint32_t* ahmax;   // [R][ah_parts] the omax of the launch that wrote ah
     uint64_t* nonfinite;     // non-finite outputs of the omax form are reported here
     int32_t nonfinite_stage;
     int32_t gather_div;      // with perm: A row (and sa entry) of slot s = perm[s] / gather_div
@@ -316,6 +316,9 @@ struct ExpertGemmArgs {
     int32_t out_tcol;        // out in column-tile order with out_rows rows
     int32_t out_rows;
     int32_t ah_tcol;         // ah in column-tile order with a_rows rows
+    int32_t ah_parts;        // parts of the launch that wrote ah
+    int32_t experts;
+    int32_t compact;         // 1: consecutive workgroups take the experts that have routes (nth_active_expert)
 };
 
 // R4: scatter-combine.

@@ -960,19 +960,42 @@ nh_status nh_moe_permute(nh_context* ctx, const int32_t* indices, size_t tokens,
 
 }  // extern "C"
 
+constexpr int kExpertWaves = 8;
+
+// Experts that evenly spread routes reach.
+static double expected_experts(size_t experts, size_t routes) {
+    return experts * (1.0 - std::pow(1.0 - 1.0 / (double)experts, (double)routes));
+}
+
+// Workgroups per expert: as many as give every CU one at the number of experts
+// that evenly spread routes reach, at least two, and no fewer than 4 N tiles
+// each (8, one per wave, when segments are longer than a 16-row block: every
+// part stages the whole segment).  A CU streams one part's weights at a time,
+// so more parts than CUs cost a second round: 8 tokens over 128 experts top-6
+// (~40 reached) in 2 / 6 / 11 / 16 parts: 55.2 / 32.4 / 36.1 / 42.4 us for
+// the up projection; 16 tokens (~68) in 2 / 3 / 6: 61.4 / 53.1 / 57.8.
+static int expert_parts(const nh_context* ctx, size_t experts, size_t routes, size_t max_rows, size_t n) {
+    const double active = expected_experts(experts, routes);
+    const int64_t ntiles = (int64_t)((n + 15) / 16), least = max_rows <= 16 ? 4 : 8;
+    int64_t parts = (int64_t)(ctx->cu_count / std::max(1.0, active));
+    parts = std::min(parts, (ntiles + least - 1) / least);
+    parts = std::min<int64_t>(parts, (int64_t)n / 4);  // the row maxima [R][parts] take the place of int8 codes [R][n]
+    return (int)std::max<int64_t>(2, parts);
+}
+
 // The expert-block kernel (slot-ordered A, kernels/moe.hip) in one of its
-// three forms; e carries the operands, this fills the launch shape.  Two
-// workgroups per expert, each owning half of the N tiles; a pass stages as
-// many 16-row blocks (up to 4) as the LDS holds next to the pass's row
-// scales, 64 row maxima and the workgroup's weight scales: every pass
-// re-streams the expert's weights.  NH_UNSUPPORTED when even one block does
+// three forms; e carries the operands, this fills the launch shape.  `parts`
+// workgroups per expert, each owning a range of its N tiles; a pass stages as
+// many 16-row blocks (up to 4, and no more than the longest segment can have:
+// max_rows) as the LDS holds next to the pass's row scales, 64 row maxima
+// and the workgroup's weight scales: every pass re-streams the expert's
+// weights.  NH_UNSUPPORTED when even one block does
 // not fit (the caller takes the grouped kernel).
 static nh_status launch_expert_gemm(nh_context* ctx, KernelId id, ExpertGemmArgs e, size_t experts, size_t n,
-                                    size_t k, nh_stream stream, nh_error* err) {
-    constexpr int kExpertWaves = 8;
+                                    size_t k, size_t routes, size_t max_rows, int parts, nh_stream stream, nh_error* err) {
     const int kt = (int)tiled_k_tiles(k);
     const int ntiles = (int)((n + 15) / 16);
-    const int tiles_per_wg = (ntiles + 1) / 2;
+    const int tiles_per_wg = (ntiles + parts - 1) / parts;
     // the weight scales arrive by 64-float direct-to-LDS rows (256 bytes
     // each, also past the workgroup's last column), so their region is a
     // whole number of rows
@@ -981,18 +1004,23 @@ static nh_status launch_expert_gemm(nh_context* ctx, KernelId id, ExpertGemmArgs
         const size_t sws_floats = ((size_t)tiles_per_wg * 16 + 63) / 64 * 64;
         return (size_t)rb * kt * 1024 + (size_t)rb * 16 * 4 + 64 * 4 + sws_floats * 4 * (e.bias ? 2 : 1);
     };
-    int row_blocks = 4;
+    int row_blocks = (int)std::min<size_t>(4, (max_rows + 15) / 16);
     while (row_blocks > 1 && expert_lds(row_blocks) > ctx->max_shared_per_block) --row_blocks;
     const size_t lds = expert_lds(row_blocks);
     if (lds > ctx->max_shared_per_block) return set_error(err, NH_UNSUPPORTED, "expert tiles exceed the LDS");
     e.N = (int)n;
     e.K = (int)k;
     e.kt = kt;
-    e.waves = 1;
+    e.parts = parts;
+    e.experts = (int)experts;
     e.streams = kExpertWaves;
     e.tiles_per_wg = tiles_per_wg;
     e.row_blocks = row_blocks;
-    return launch(ctx, id, 2u, (unsigned)(64 * kExpertWaves), lds, stream, e, err, (unsigned)experts);
+    // the search for the experts with routes only where many have none (512
+    // tokens over 128 experts, where it finds the same order: 0.5 us per launch)
+    e.compact = expected_experts(experts, routes) < 0.9 * (double)experts;
+    const size_t slots = e.compact ? std::min(experts, routes) : experts;
+    return launch(ctx, id, (unsigned)(parts * slots), (unsigned)(64 * kExpertWaves), lds, stream, e, err);
 }
 
 // Whether the MoE layer's two projections run as the fused expert-block
@@ -1043,7 +1071,8 @@ static nh_status moe_grouped_gemm(nh_context* ctx, const int8_t* aq, const float
         e.out = out;
         e.a_rows = (int)a_rows;
         e.relu2 = relu2 ? 1 : 0;
-        st = launch_expert_gemm(ctx, K_EXPERT_GEMM, e, experts, n, k, stream, err);
+        st = launch_expert_gemm(ctx, K_EXPERT_GEMM, e, experts, n, k, routes, routes, expert_parts(ctx, experts, routes, routes, n), stream,
+                                err);
         if (st != NH_UNSUPPORTED) return st;
         clear_error(err);
     }
@@ -1251,7 +1280,8 @@ static nh_status moe_forward(nh_context* ctx, const void* x, nh_dtype x_dtype, c
         // the layer's intermediate); the down projection requantizes h per
         // row while it stages it (the codes and scales of
         // nh_quantize_rows_i8 on h), then adds its bias
-        uint32_t* hmax = (uint32_t*)(ws + off[8]);  // [R][2]
+        const int parts_up = expert_parts(ctx, experts, R, tokens, inter);
+        uint32_t* hmax = (uint32_t*)(ws + off[8]);  // [R][parts_up]
         ExpertGemmArgs up{};
         up.aq = xq;
         up.sa = sx;
@@ -1271,18 +1301,20 @@ static nh_status moe_forward(nh_context* ctx, const void* x, nh_dtype x_dtype, c
         up.omax = hmax;
         up.nonfinite = nonfinite;
         up.nonfinite_stage = kStageIntermediate;
-        if ((st = launch_expert_gemm(ctx, K_EXPERT_GEMM_OMAX, up, experts, inter, hidden, stream, err))) return st;
+        if ((st = launch_expert_gemm(ctx, K_EXPERT_GEMM_OMAX, up, experts, inter, hidden, R, tokens, parts_up, stream, err))) return st;
         ExpertGemmArgs down{};
         down.ah = h;
         down.ah_tcol = 1;
         down.ahmax = hmax;
+        down.ah_parts = parts_up;
         down.offsets = offsets;
         down.w = w_down;
         down.sw = s_down;
         down.bias = b.down;
         down.out = d;
         down.a_rows = (int)R;
-        if ((st = launch_expert_gemm(ctx, K_EXPERT_GEMM_QA, down, experts, hidden, inter, stream, err))) return st;
+        if ((st = launch_expert_gemm(ctx, K_EXPERT_GEMM_QA, down, experts, hidden, inter, R, tokens,
+                                     expert_parts(ctx, experts, R, tokens, hidden), stream, err))) return st;
     } else {
         if ((st = moe_grouped_gemm(ctx, xq, sx, 0, top_k, offsets, perm, R, R, experts, w_up, s_up, b.up, inter,
                                    hidden, 1, h, stream, err)))
