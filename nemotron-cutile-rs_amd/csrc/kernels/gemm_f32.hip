@@ -14,8 +14,6 @@
 // For the MoE router (moe.rs:185-188, a dense f32 LinearProjection) the lhs
 // may be bf16 (widened exactly to f32 on load) and a bias may follow the
 // rounding to f32, as project_into adds it (linear.rs:330-336).
-#include <type_traits>
-
 #include "nh_device.h"
 
 using namespace nh;
@@ -102,137 +100,219 @@ extern "C" __global__ __launch_bounds__(256) void nh_gemm_f32_kernel(GemmF32Args
 // B[k][j] of block b, D lane 16 i + 4 b + j holds D[i][j] of block b: four
 // 4 x 4 blocks per wave.
 //
-// A workgroup of 4 waves owns 16 x 16 outputs: wave w the rows 4w..4w+3 and,
-// as its blocks b, the columns 4b..4b+3.  K advances in chunks of 128 through
-// LDS (f32, widened as an operand is read; double buffered, the loads of the
-// next two chunks in flight while the current one runs).  A chunk's operands
-// are read into registers before its chain, so the LDS latency is paid once
-// per chunk.  k past K, rows past M and columns past N are zeros: an added
-// fma(0, 0, acc) leaves acc unchanged, as acc starts at +0.0 and a k-ordered
-// sum of products that starts there is never -0.0.  One chain of 64 outputs
-// per wave takes ~21 cycles per 4-k step (the MFMA's dependent latency; its
-// issue rate is one per 16 cycles), against ~40 cycles per single k step for
-// a lane-per-output FMA chain.
+// A workgroup owns 16 x 16 outputs and has two roles.  Chain wave w (0..3) runs
+// the rows 4w..4w+3 with, as its blocks b, the columns 4b..4b+3: one chain of
+// 64 outputs, 21 cycles per 4-k step (the MFMA's dependent latency; its issue
+// rate is one per 16), and does nothing but operand reads and MFMAs.  Staging
+// waves (4, 5: lhs, 6, 7: rhs) load the operands, widen them to f64 once and
+// write them to LDS in the chain's order, two steps of a lane side by side, so
+// a chain wave reads two steps' operands with two 16-byte reads.  With the
+// loads and the widening in the chain waves a step took ~56 cycles.
+// K advances in chunks of 64 through three LDS buffers (55 KiB: two workgroups
+// per CU).  Barrier c says that chunk c is written; the chain waves pass it
+// halfway through chunk c - 1 and read four step pairs ahead, so neither the
+// barrier nor the LDS latency interrupts the chain.  The staging waves write
+// chunk c + 1 after barrier c, into the buffer of chunk c - 2, which the chain
+// waves have finished by then; their loads run six chunks ahead (a chunk is
+// ~0.15 us of chain, a load from HBM over 1 us).
+// k past K, rows past M and columns past N are zeros: an added fma(0, 0, acc)
+// leaves acc unchanged, as acc starts at +0.0 and a k-ordered sum of products
+// that starts there is never -0.0.
+// Bound by the chain: 672 steps at K = 2688 are 6 us, the launch and the first
+// loads ~6 more.  Measured: 8 x 2688 x 128 23.4 -> 14.2 us, 512 x 2688 x 128
+// 25.0 -> 19.4, 100 x 4096 x 60 34.4 -> 24.0, 2048 x 4096 x 128 (four rounds, the
+// MFMA pipes busy) 84.2 -> 82.0.  Chunks of 128 in 108 KiB were as fast on one
+// round and 93 us on four.
 //
 // Loads go through buffer resources over the whole operands (wave-uniform;
 // the launch keeps both below 2^31 bytes), positions past the matrix sent out
-// of range so they read zeros with no branch, and every fetch issues the same
-// loads, so the waits before a chunk is staged count exactly the younger
-// fetch's loads.  VEC (16-byte aligned operands, K a multiple of 8 for bf16 or
-// 4 for f32, N a multiple of 4): 16-byte loads, 3 or 4 per thread and chunk;
-// otherwise one load per value.
+// of range so they read zeros with no branch.  VEC (16-byte aligned lhs, K a
+// multiple of 8 for bf16 or 4 for f32): 16-byte lhs loads; otherwise one load
+// per value.
 namespace {
 
+constexpr int kF32Chunk = 64;                   // k per chunk: 8 pairs of 4-k steps
+constexpr int kF32Ahead = 6;                     // chunks of operands in flight per staging thread
+constexpr int kF32Pairs = kF32Chunk / 8;
+constexpr int kF32APair = 320;                  // bytes of a step pair of 4 rows: 256, padded against bank conflicts
+constexpr int kF32AGroup = kF32Pairs * kF32APair;
+constexpr int kF32ABytes = 4 * kF32AGroup;
+constexpr int kF32Buffer = kF32ABytes + kF32Pairs * 1024;  // A of the 4 row groups, then B
+static_assert(3 * kF32Buffer == kGemmF32MfmaLds, "the host's LDS size");
+
+typedef double nh_v2d __attribute__((ext_vector_type(2)));
+
+// One staging thread's operand (A: row t / 8, the step pair t % 8, i.e. 8
+// consecutive k; B: column t % 16, the step pair t / 16), chunk by chunk.
+// Offsets past the matrix get bit 31 (operands are below 2^31 bytes), by
+// arithmetic: a select becomes a branch around the load, and then every wait
+// a wait for all loads (23 us instead of 14 at 8 x 2688 x 128).
+__device__ __forceinline__ uint32_t past_end(int v, int end) { return (uint32_t)((end - 1 - v) >> 31) & 0x80000000u; }
+
 template <bool BF16, bool VEC>
-__device__ __forceinline__ void gemm_f32_mfma(const GemmF32Args& a) {
-    constexpr int KC = 128;
-    __shared__ float As[2][16][KC + 4];  // [row][k]; the pad puts the 16 rows of a read on distinct banks
-    __shared__ float Bs[2][KC][16];      // [k][column]
-    const int t = threadIdx.x, lane = t & 63;
-    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int64_t M = a.M, K = a.K, N = a.N;
-    const int64_t tiles_n = (N + 15) / 16;
-    const int64_t m0 = (int64_t)(blockIdx.x / tiles_n) * 16, n0 = (int64_t)(blockIdx.x % tiles_n) * 16;
-    // staging roles: A row t / 16, k (t % 16) * 8 .. + 7; B k-rows t / 4 and
-    // t / 4 + 64, columns (t % 4) * 4 .. + 3
-    const int64_t am = m0 + (t >> 4), ak = (t & 15) * 8, bk = t >> 2, bn = n0 + (t & 3) * 4;
-    constexpr uint32_t esz = BF16 ? 2u : 4u;
-    const __amdgpu_buffer_rsrc_t rA = make_rsrc(a.lhs, (uint32_t)(M * K * esz));
-    const __amdgpu_buffer_rsrc_t rB = make_rsrc(a.rhs, (uint32_t)(K * N * 4));
-    const uint32_t oor = (uint32_t)kOutOfRange;
-    float ra[2][8], rb[2][8];  // chunks c + 1 and c + 2 in flight
-    auto fetch = [&](int64_t k0, float (&ra)[8], float (&rb)[8]) {
-        const int64_t gk = k0 + ak;
-        const uint32_t abase = (uint32_t)((am * K + gk) * esz);
-        if constexpr (VEC && BF16) {
-            const v4i v = buffer_load16(rA, am < M && gk < K ? abase : oor);
+struct StageA {
+    static constexpr int kRegs = VEC && BF16 ? 4 : 8;
+    static constexpr uint32_t esz = BF16 ? 2u : 4u;
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t start;
+    int k0, K, lds0;
+    __device__ StageA(const GemmF32Args& a, int t, int64_t m0, int64_t)
+        : r(make_rsrc(a.lhs, (uint32_t)a.M * (uint32_t)a.K * esz)), k0(8 * (t & 7)), K((int)a.K) {
+        const int row = t >> 3, m = (int)m0 + row;
+        start = ((uint32_t)m * (uint32_t)K + (uint32_t)k0) * esz | past_end(m, (int)a.M);
+        lds0 = (row >> 2) * kF32AGroup + (t & 7) * kF32APair + (row & 3) * 16;
+    }
+    __device__ void fetch(int c, uint32_t (&v)[kRegs]) const {
+        const uint32_t base = start + (uint32_t)(c * kF32Chunk) * esz;
+        const int k = c * kF32Chunk + k0;
+        if constexpr (VEC) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                ra[2 * e] = f32_from_bits((uint32_t)v[e] << 16);
-                ra[2 * e + 1] = f32_from_bits((uint32_t)v[e] & 0xffff0000u);
-            }
-        } else if constexpr (VEC) {
+            for (int h = 0; h < kRegs / 4; ++h) {
+                const v4i x = buffer_load16(r, (int)((base + 16u * h) | past_end(k + 4 * h, K)));
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const v4i v = buffer_load16(rA, am < M && gk + 4 * h < K ? abase + 16u * h : oor);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) ra[4 * h + e] = f32_from_bits((uint32_t)v[e]);
+                for (int e = 0; e < 4; ++e) v[4 * h + e] = (uint32_t)x[e];
             }
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const uint32_t off = am < M && gk + e < K ? abase + esz * e : oor;
-                ra[e] = BF16 ? f32_from_bits((uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rA, off, 0, 0) << 16)
-                             : f32_from_bits(__builtin_amdgcn_raw_buffer_load_b32(rA, off, 0, 0));
+                const uint32_t off = (base + esz * e) | past_end(k + e, K);
+                v[e] = BF16 ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0)
+                            : (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
             }
         }
+    }
+    static __device__ double value(const uint32_t (&v)[kRegs], int e) {
+        if constexpr (!BF16) return (double)f32_from_bits(v[e]);
+        else if constexpr (VEC) return (double)f32_from_bits((e & 1) ? v[e >> 1] & 0xffff0000u : v[e >> 1] << 16);
+        else return (double)f32_from_bits(v[e] << 16);
+    }
+    // k = 8 pair + 4 h + kk: step 2 pair + h, the MFMA's k index kk
+    __device__ void store(int8_t* buf, const uint32_t (&v)[kRegs]) const {
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int64_t gkb = k0 + bk + 64 * h;
-            const uint32_t bbase = (uint32_t)((gkb * N + bn) * 4);
-            if constexpr (VEC) {
-                const v4i v = buffer_load16(rB, gkb < K && bn < N ? bbase : oor);
+        for (int kk = 0; kk < 4; ++kk) *(nh_v2d*)(buf + lds0 + kk * 64) = nh_v2d{value(v, kk), value(v, kk + 4)};
+    }
+};
+
+struct StageB {
+    static constexpr int kRegs = 8;
+    __amdgpu_buffer_rsrc_t r;
+    uint32_t start, step;
+    int lds0;
+    __device__ StageB(const GemmF32Args& a, int t, int64_t, int64_t n0)
+        : r(make_rsrc(a.rhs, (uint32_t)a.K * (uint32_t)a.N * 4u)), step((uint32_t)a.N * 4u) {
+        const int n = (int)n0 + (t & 15);
+        start = (8u * (uint32_t)(t >> 4) * (uint32_t)a.N + (uint32_t)n) * 4u | past_end(n, (int)a.N);
+        lds0 = kF32ABytes + (t >> 4) * 1024 + (t & 15) * 16;
+    }
+    __device__ void fetch(int c, uint32_t (&v)[kRegs]) const {  // (k past K: past the end of rhs)
+        uint32_t off = start + (uint32_t)(c * kF32Chunk) * step;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) rb[4 * h + e] = f32_from_bits((uint32_t)v[e]);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    rb[4 * h + e] = f32_from_bits(
-                        __builtin_amdgcn_raw_buffer_load_b32(rB, gkb < K && bn + e < N ? bbase + 4u * e : oor, 0, 0));
-            }
+        for (int e = 0; e < 8; ++e) {
+            v[e] = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+            off += step;
         }
+    }
+    __device__ void store(int8_t* buf, const uint32_t (&v)[kRegs]) const {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+            *(nh_v2d*)(buf + lds0 + kk * 256) =
+                nh_v2d{(double)f32_from_bits(v[kk]), (double)f32_from_bits(v[kk + 4])};
+    }
+};
+
+template <class Stage>
+__device__ __forceinline__ void gemm_f32_stage(const Stage& s, int8_t* lds, int nc) {
+    uint32_t v[kF32Ahead][Stage::kRegs];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < kF32Ahead; ++u) {  // (chunks past the last: zeros)
+        s.fetch(u, v[u]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    int buf = 0;
+    for (int c = 0; c < nc; c += kF32Ahead) {
+#pragma unroll
+        for (int u = 0; u < kF32Ahead; ++u) {
+            if (c + u >= nc) break;  // uniform
+            s.store(lds + buf * kF32Buffer, v[u]);
+            s.fetch(c + u + kF32Ahead, v[u]);
+            lds_publish();  // barrier c + u
+            buf = buf == 2 ? 0 : buf + 1;
+        }
+    }
+}
+
+__device__ __forceinline__ void gemm_f32_chain(const GemmF32Args& a, const int8_t* lds, int64_t m0, int64_t n0, int nc) {
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (m0 + 4 * w >= a.M) {  // no rows (uniform): the barriers only
+        for (int c = 0; c < nc; ++c) lds_barrier();
+        return;
+    }
+    // lane l: A[row l % 4][k l / 16], B[k l / 16][column l % 16]
+    const int8_t* pa = lds + w * kF32AGroup + (lane >> 4) * 64 + (lane & 3) * 16;
+    const int8_t* pb = lds + kF32ABytes + lane * 16;
+    constexpr int AHEAD = 4;  // step pairs read ahead
+    nh_v2d av[AHEAD], bv[AHEAD];
+    auto read = [&](int buf, int p) {
+        av[p % AHEAD] = *(const nh_v2d*)(pa + buf * kF32Buffer + p * kF32APair);
+        bv[p % AHEAD] = *(const nh_v2d*)(pb + buf * kF32Buffer + p * 1024);
     };
-    // MFMA operand roles of this lane
-    const int rk = lane >> 4, arow = 4 * w + (lane & 3), bcol = 4 * ((lane >> 2) & 3) + (lane & 3);
     double acc = 0.0;
-    // chunk at k0 from LDS buffer B (a constant, so the register sets are
-    // not indexed at run time)
-    auto chunk = [&](int64_t k0, auto bufc) {
-        constexpr int B = decltype(bufc)::value;
+    lds_barrier();  // chunk 0
 #pragma unroll
-        for (int e = 0; e < 8; ++e) As[B][t >> 4][ak + e] = ra[B][e];
+    for (int p = 0; p < AHEAD; ++p) read(0, p);
+    int buf = 0;
+    for (int c = 0; c < nc; ++c) {
+        const int next = buf == 2 ? 0 : buf + 1;
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) Bs[B][bk + 64 * h][(t & 3) * 4 + e] = rb[B][4 * h + e];
-        __syncthreads();
-        if (k0 + 2 * KC < K) fetch(k0 + 2 * KC, ra[B], rb[B]);  // uniform
-        float av[KC / 4], bv[KC / 4];
-#pragma unroll
-        for (int st = 0; st < KC / 4; ++st) {
-            av[st] = As[B][arow][4 * st + rk];
-            bv[st] = Bs[B][4 * st + rk][bcol];
+        for (int p = 0; p < kF32Pairs; ++p) {
+            if (p == kF32Pairs / 2 && c + 1 < nc) lds_barrier();  // chunk c + 1
+            const nh_v2d x = av[p % AHEAD], y = bv[p % AHEAD];
+            acc = __builtin_amdgcn_mfma_f64_4x4x4f64(x[0], y[0], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f64_4x4x4f64(x[1], y[1], acc, 0, 0, 0);
+            // (after the last chunk the reads are of an older one, and unused)
+            if (p + AHEAD < kF32Pairs) read(buf, p + AHEAD);
+            else read(next, p + AHEAD - kF32Pairs);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);  // the reads go out ahead of the chain
-#pragma unroll
-        for (int st = 0; st < KC / 4; ++st)
-            acc = __builtin_amdgcn_mfma_f64_4x4x4f64((double)av[st], (double)bv[st], acc, 0, 0, 0);
-    };
-    fetch(0, ra[0], rb[0]);
-    if (KC < K) fetch(KC, ra[1], rb[1]);
-    for (int64_t k0 = 0; k0 < K; k0 += 2 * KC) {
-        chunk(k0, std::integral_constant<int, 0>{});
-        if (k0 + KC < K) chunk(k0 + KC, std::integral_constant<int, 1>{});  // uniform
+        buf = next;
     }
     // D lane 16 i + 4 b + j: output (4w + i, 4b + j)
     const int64_t gm = m0 + 4 * w + (lane >> 4), gn = n0 + 4 * ((lane >> 2) & 3) + (lane & 3);
-    if (gm < M && gn < N) a.out[gm * N + gn] = a.bias ? (float)acc + a.bias[gn] : (float)acc;
+    if (gm < a.M && gn < a.N) a.out[gm * a.N + gn] = a.bias ? (float)acc + a.bias[gn] : (float)acc;
+}
+
+template <bool BF16, bool VEC>
+__device__ __forceinline__ void gemm_f32_mfma(const GemmF32Args& a, int8_t* lds) {
+    const int64_t tiles_n = (a.N + 15) / 16;
+    const int64_t m0 = (int64_t)(blockIdx.x / tiles_n) * 16, n0 = (int64_t)(blockIdx.x % tiles_n) * 16;
+    const int nc = (int)((a.K + kF32Chunk - 1) / kF32Chunk);
+    if (threadIdx.x < 256)
+        gemm_f32_chain(a, lds, m0, n0, nc);
+    else if (threadIdx.x < 384)
+        gemm_f32_stage(StageA<BF16, VEC>(a, threadIdx.x - 256, m0, n0), lds, nc);
+    else
+        gemm_f32_stage(StageB(a, threadIdx.x - 384, m0, n0), lds, nc);
 }
 
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(256) void nh_gemm_f32_mfma_kernel(GemmF32Args a) {
-    gemm_f32_mfma<false, true>(a);
+extern "C" __global__ __launch_bounds__(512) void nh_gemm_f32_mfma_kernel(GemmF32Args a) {
+    extern __shared__ __align__(1024) int8_t smem[];
+    gemm_f32_mfma<false, true>(a, smem);
 }
 
-extern "C" __global__ __launch_bounds__(256) void nh_gemm_f32_mfma_bf16_kernel(GemmF32Args a) {
-    gemm_f32_mfma<true, true>(a);
+extern "C" __global__ __launch_bounds__(512) void nh_gemm_f32_mfma_bf16_kernel(GemmF32Args a) {
+    extern __shared__ __align__(1024) int8_t smem[];
+    gemm_f32_mfma<true, true>(a, smem);
 }
 
-// Any alignment, K and N: one load per value.
-extern "C" __global__ __launch_bounds__(256) void nh_gemm_f32_mfma_any_kernel(GemmF32Args a) {
+// Any alignment and K: one load per value.
+extern "C" __global__ __launch_bounds__(512) void nh_gemm_f32_mfma_any_kernel(GemmF32Args a) {
+    extern __shared__ __align__(1024) int8_t smem[];
     if (a.lhs_bf16)
-        gemm_f32_mfma<true, false>(a);
+        gemm_f32_mfma<true, false>(a, smem);
     else
-        gemm_f32_mfma<false, false>(a);
+        gemm_f32_mfma<false, false>(a, smem);
 }

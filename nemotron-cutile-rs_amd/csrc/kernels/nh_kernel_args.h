@@ -229,6 +229,9 @@ struct GemmDirectArgs {
     int32_t pad_;
 };
 
+// Dynamic LDS of the f64 matrix-core GEMM (gemm_f32.hip): three chunks of 64 k.
+constexpr int kGemmF32MfmaLds = 3 * (4 * 8 * 320 + 8 * 1024);
+
 // R1: sigmoid top-k routing, one wave per token.
 struct RouteArgs {
     const float* scores;  // [T][E]

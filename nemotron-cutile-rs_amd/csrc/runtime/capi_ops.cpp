@@ -639,8 +639,8 @@ int nh_supports_gemm_f32(size_t m, size_t k, size_t n) {
 // lane, f64 FMAs) while those tiles fill every CU, else 16 x 16 outputs per
 // workgroup on the f64 matrix cores (v_mfma_f64_4x4x4f64 chains), so a narrow
 // output such as the MoE router's 128 experts still spreads its k-ordered
-// chains over the chip (512 x 2688 x 128: 24.1 us against 52.3 us for one
-// output per lane on f64 FMAs; 2048 x 4096 x 128: 80 against 180 us;
+// chains over the chip (512 x 2688 x 128: 19.4 us against 52.3 us for one
+// output per lane on f64 FMAs; 2048 x 4096 x 128: 82 against 180 us;
 // 512 x 4096 x 4096 stays on the 64 x 64 tiles: 531 us against 628 on the
 // matrix cores).
 static nh_status launch_gemm_f32(nh_context* ctx, const GemmF32Args& a, nh_stream stream, nh_error* err) {
@@ -655,9 +655,9 @@ static nh_status launch_gemm_f32(nh_context* ctx, const GemmF32Args& a, nh_strea
     if (lhs_bytes >= 0x7ffffff0u || rhs_bytes >= 0x7ffffff0u)  // the kernels' out-of-range offset
         return launch(ctx, K_GEMM_F32, (unsigned)((a.N + 63) / 64), 256, 0, stream, a, err,
                       (unsigned)((a.M + 63) / 64));
-    const bool vec = aligned16(a.lhs) && aligned16(a.rhs) && a.K % (a.lhs_bf16 ? 8 : 4) == 0 && a.N % 4 == 0;
+    const bool vec = aligned16(a.lhs) && a.K % (a.lhs_bf16 ? 8 : 4) == 0;
     const KernelId id = !vec ? K_GEMM_F32_MFMA_ANY : a.lhs_bf16 ? K_GEMM_F32_MFMA_BF16 : K_GEMM_F32_MFMA;
-    return launch(ctx, id, (unsigned)(((a.M + 15) / 16) * ((a.N + 15) / 16)), 256, 0, stream, a, err);
+    return launch(ctx, id, (unsigned)(((a.M + 15) / 16) * ((a.N + 15) / 16)), 512, kGemmF32MfmaLds, stream, a, err);
 }
 
 nh_status nh_gemm_f32(nh_context* ctx, const float* lhs, size_t lhs_len, const float* rhs, size_t rhs_len, size_t m,
