@@ -28,7 +28,6 @@ using namespace nh;
 
 namespace {
 
-typedef uint32_t nh_v2u __attribute__((ext_vector_type(2)));
 typedef float nh_v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kDirectWaves = 4;
@@ -160,7 +159,6 @@ __device__ __forceinline__ void direct_tile(const GemmDirectArgs& d, int8_t* lds
     constexpr int PER = kDirectPhase / W;
     const int esz = a.out_dtype == DT_BF16 ? 2 : 4;
     const int64_t ldo = a.ldo;
-    const bool aligned = ((((uint64_t)a.out) | ((uint64_t)ldo * esz)) & (uint64_t)(4 * esz - 1)) == 0;
 #pragma unroll
     for (int p0 = 0; p0 < F; p0 += kDirectPhase) {
         if (p0) __syncthreads();
@@ -194,13 +192,9 @@ __device__ __forceinline__ void direct_tile(const GemmDirectArgs& d, int8_t* lds
                 if (a.relu2) y[r] = relu2(y[r]);
             }
             if (m >= M) continue;
-            int8_t* o = (int8_t*)a.out + ((int64_t)m * ldo + n) * esz;
-            if (aligned && n + 3 < N) {
-                if (esz == 2)
-                    *(nh_v2u*)o = nh_v2u{f32x2_to_bf16x2(y[0], y[1]), f32x2_to_bf16x2(y[2], y[3])};
-                else
-                    *(nh_v4f*)o = nh_v4f{y[0], y[1], y[2], y[3]};
-            } else {  // the matrix edge, or unaligned rows
+            if (n + 3 < N) {
+                store_cols4((int8_t*)a.out + ((int64_t)m * ldo + n) * esz, y, esz == 2);
+            } else {  // the matrix edge
 #pragma unroll 1
                 for (int r = 0; r < 4 && n + r < N; ++r) {
                     store_out(a.out, (int64_t)m * ldo + n + r, y[0], a.out_dtype);

@@ -148,6 +148,18 @@ __device__ __forceinline__ uint32_t f32x2_to_bf16x2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, nh_bf16x2));
 }
 
+// Four consecutive outputs of one row as one 8-byte (bf16) or 16-byte (f32)
+// store at an address aligned to the element only: vector stores to global
+// memory take any alignment (a row of odd length starts anywhere).
+__device__ __forceinline__ void store_cols4(void* p, const float (&y)[4], bool bf16) {
+    if (bf16) {
+        const uint32_t v[2] = {f32x2_to_bf16x2(y[0], y[1]), f32x2_to_bf16x2(y[2], y[3])};
+        __builtin_memcpy(p, v, 8);
+    } else {
+        __builtin_memcpy(p, y, 16);
+    }
+}
+
 // Largest bf16 magnitude of the 8 values of one 16-byte load, as its 15-bit
 // pattern (sign cleared).  Magnitude bit patterns order like the values, and
 // infinities and NaNs (0x7f80 and above) order above every finite value, so

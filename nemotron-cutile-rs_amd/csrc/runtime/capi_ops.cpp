@@ -146,8 +146,12 @@ nh_status launch_quantize(nh_context* ctx, const void* x, nh_dtype dtype, size_t
                        act_p > 0 ? act_p : (int)rows, gather_div, gather, nonfinite, nonfinite_stage, 0};
     // the GEMM's A tiles for many rows of up to 512 chunks: 8 rows per
     // workgroup, whole 128-byte lines per store (M = 2048 linear layer,
-    // 4096 -> 4096: 45.6-45.8 us against 46.1-46.7 with the wave kernel)
-    if (vec && q_act && act_p == 16 && !gather && rows > 16 && row_bytes <= 512 * 16) {
+    // 4096 -> 4096: 45.6-45.8 us against 46.1-46.7 with the wave kernel).
+    // Fewer rows leave CUs idle that way, and a workgroup per row is faster:
+    // 77 x 4096 bf16 with its product 15.8 against 17.7 us, 800 rows 19.3
+    // against 20.6; half-length rows only below 512 (800 x 1024 f32 11.0 / 10.4).
+    const size_t tile_rows = (row_bytes > 256 * 16 ? 4 : 2) * (size_t)ctx->cu_count;
+    if (vec && q_act && act_p == 16 && !gather && rows >= tile_rows && row_bytes <= 512 * 16) {
         const size_t lds = 8 * 64 * tiled_k_tiles(cols);
         return launch(ctx, K_QUANTIZE_TILES, (unsigned)((rows + 7) / 8), 512, lds, stream, a, err);
     }
@@ -158,8 +162,10 @@ nh_status launch_quantize(nh_context* ctx, const void* x, nh_dtype dtype, size_t
     if (vec && row_bytes <= 512 * 16 && rows >= 1024)
         return launch(ctx, K_QUANTIZE_ROWS_WAVE, (unsigned)((rows + 3) / 4), 256, 0, stream, a, err);
     // a few rows longer than a 256-thread workgroup holds in registers
-    // (1024 chunks): 1024 threads per row, one round trip to memory
-    if (vec && row_bytes > 1024 * 16 && rows <= 256)
+    // (1024 chunks; 2816 in the form below): 1024 threads per row, one round
+    // trip to memory (500 x 21504 f32 with its product 69.7 against 72.6 us,
+    // 1000 rows 83.5 / 86.7, 2048 rows 115.8 / 115.2)
+    if (vec && row_bytes > 1024 * 16 && rows <= (row_bytes > 2816 * 16 ? 4 : 1) * (size_t)ctx->cu_count)
         return launch(ctx, K_QUANTIZE_ROWS_LONG, (unsigned)rows, 1024, 0, stream, a, err);
     // many rows of 1025..2816 chunks: the whole row in a 256-thread workgroup's
     // registers, read once (2048 x 21504 bf16: 3 us less)
@@ -195,7 +201,7 @@ nh_status launch_gemv(nh_context* ctx, const int8_t* xq, const float* sx, const 
 }
 
 // The persistent 256 x 224 GEMM (gemm_persistent.hip) when its contract
-// holds and its tiles fill whole rounds of CUs with less work per CU than the
+// holds and its tiles fill rounds of CUs with less work per CU than the
 // loader-wave kernel's 256 x 128 tiles: rounds x tile area (the 21504-wide
 // up projection at M = 2048: 3 rounds of 256 x 224 against 5.5 of 256 x 128;
 // measured 201-203 against 231-236 us).
@@ -213,7 +219,9 @@ bool use_persistent_224(const nh_context* ctx, const void* xq, const float* sx, 
     const int64_t cu = ctx->cu_count, tm = (M + 255) / 256;
     const int64_t tiles_p = tm * ((N + 223) / 224), tiles_o = tm * ((N + 127) / 128);
     const int64_t work_p = (tiles_p + cu - 1) / cu * 224, work_o = (tiles_o + cu - 1) / cu * 128;
-    return tiles_p >= cu && work_p < work_o;
+    // (one round on at least half of the CUs: 500 x 21504 x 4096, 192 tiles,
+    // 55.9 us against 61.6 for 256 + 160 smaller ones; 768 x 16384 x 4096 60.7 / 78.3)
+    return 2 * tiles_p >= cu && work_p < work_o;
 }
 
 // The LDS-tiled G3 kernels (gemm.hip) on tiled A, largest first.
@@ -232,24 +240,44 @@ int64_t gemm_tiles(const GemmCfg& c, int M, int N) {
     return (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
 }
 
-// The largest whose tiles fill every CU, else 64 x 64 (the most tiles); null
-// when the LDS holds none.
-const GemmCfg* tiled_gemm_cfg(const nh_context* ctx, int M, int N) {
-    for (const GemmCfg& c : kTiledCfgs)
-        if (gemm_tiles(c, M, N) >= ctx->cu_count && c.lds <= ctx->max_shared_per_block) return &c;
-    return kTiledCfgs[3].lds <= ctx->max_shared_per_block ? &kTiledCfgs[3] : nullptr;
+// Time in us of tile choice `at` on cold weights: a launch, and per round of
+// workgroups an epilogue and what the kernel's stage loop takes per 64-deep K
+// tile, more with more of the CUs busy (their clock, and the weight stream).
+// The larger tiles have a CU to themselves, so their rounds are whole (256 x
+// 128: a last round at most half full runs as 128 x 128 tiles); two or three of
+// the smaller ones share one.  Fitted to 342 shapes of 17..2048 rows, 1024..
+// 16384 columns and K = 1024..8192 (each to 7-12% r.m.s.).
+double tiled_gemm_us(const nh_context* ctx, int at, int M, int N, int kt) {
+    const int64_t t = gemm_tiles(kTiledCfgs[at], M, N), cu = ctx->cu_count;
+    const double whole = (double)((t + cu - 1) / cu), avg = std::max(1.0, (double)t / cu);
+    const double fill = std::min(1.0, (double)t / cu);
+    switch (at) {
+    case 0: {
+        const double rounds = t > cu && t % cu != 0 && t % cu <= cu / 2 ? (double)(t / cu) + 0.62 : whole;
+        return -0.35 + rounds * (8.35 + kt * (0.251 + 0.167 * fill));
+    }
+    case 1: return 1.63 + whole * (3.96 + kt * (0.197 + 0.064 * fill));
+    case 2: return 3.32 + 1.17 * avg + kt * (0.031 * avg + whole * (0.144 + 0.013 * fill));
+    default: return 3.79 + kt * (0.042 * avg + whole * (0.147 - 0.047 * fill));
+    }
 }
 
-// The time of that choice in us (cold weights; fitted with plan_direct): a
-// launch and, per round of workgroups and 64-deep K tile, what the kernel's
-// stage loop takes whatever the tile holds.
-double tiled_gemm_us(const nh_context* ctx, int M, int N, int kt) {
-    static const double launch_us[] = {5.0, 4.5, 3.5, 3.0}, kt_us[] = {0.467, 0.292, 0.255, 0.217},
-                        fill[] = {1.0, 0.9, 0.85, 0.8};
-    const GemmCfg* c = tiled_gemm_cfg(ctx, M, N);
-    if (!c) return 1e30;
-    const int at = (int)(c - kTiledCfgs);
-    return launch_us[at] + kt_us[at] * kt * std::max(1.0, fill[at] * (double)gemm_tiles(*c, M, N) / ctx->cu_count);
+// The fastest of them by that model, and its time; -1 when the LDS holds none.
+// (The largest tile that fills every CU, which the choice once was, is far off
+// where its tiles leave a second round nearly empty: 1024 x 4099 x 2688 on 264
+// tiles of 128 x 128 32.0 us, on 132 of 256 x 128 24.9; 613 x 10304 x 2688 36.7 / 28.3.)
+int tiled_gemm_cfg(const nh_context* ctx, int M, int N, int kt, double* us) {
+    int best = -1;
+    *us = 1e30;
+    for (int at = 0; at < 4; ++at) {
+        if (kTiledCfgs[at].lds > ctx->max_shared_per_block) continue;
+        const double u = tiled_gemm_us(ctx, at, M, N, kt);
+        if (best < 0 || u < *us) {
+            best = at;
+            *us = u;
+        }
+    }
+    return best;
 }
 
 // The register-direct GEMM (gemm_direct.hip): its tile for a shape, and the
@@ -261,11 +289,10 @@ struct DirectPlan {
     double us;
 };
 
-// Fitted to 216 shapes of 17..512 rows, 1024..16384 columns and K = 1024..8192
-// (cold weights): a launch, then per round of workgroups an epilogue, and
-// per K tile the fragments through the CU's load path (66 KiB per us), or the
+// Fitted to the same shapes: a launch, then per round of workgroups an epilogue, and
+// per K tile the fragments through the CU's load path (80 KiB per us), or the
 // weights from HBM (5.6 TB/s) where that is longer.  Against the LDS tiles
-// (tiled_gemm_us), both sides measured at M x N x K: 17 x 2688 x 2688 5.5 / 11.8
+// (tiled_gemm_cfg), both sides measured at M x N x K: 17 x 2688 x 2688 5.5 / 11.8
 // us, 77 x 6144 x 4096 11.5 / 15.8, 400 x 2688 x 4096 15.5 / 20.9, 64 x 16384 x
 // 1024 7.8 / 6.8, 512 x 16384 x 4096 49.2 / 36.2.
 DirectPlan plan_direct(const nh_context* ctx, int M, int N, int kt, bool w4) {
@@ -280,10 +307,13 @@ DirectPlan plan_direct(const nh_context* ctx, int M, int N, int kt, bool w4) {
         const int mr = (mtiles + groups - 1) / groups;
         const int64_t tn = (N + 16 * nr - 1) / (16 * nr), wgs = tn * groups;
         if ((tn + 7) / 8 * 8 * groups > kMaxGrid) continue;
-        const double rounds = std::max(1.0, 1.15 * (double)wgs / cu);
-        const double load = rounds * kt * (mr + (w4 ? 0.5 : 1.0) * nr) / 66.0;
+        // between whole rounds (a CU with two workgroups shares its load path)
+        // and the average
+        const double rounds = 0.5 * std::ceil((double)wgs / cu) + 0.5 * std::max(1.0, (double)wgs / cu);
+        const double load = rounds * kt * (mr + (w4 ? 0.5 : 1.0) * nr) / 80.0 *
+                            (0.85 + 0.2 * std::min(1.0, (double)wgs / cu));
         const double hbm = (double)N * kt * (w4 ? 32 : 64) / 5.6e6;
-        const double us = 2.2 + rounds * (1.2 + 0.07 * mr * nr) + std::max(load, hbm);
+        const double us = 2.0 + rounds * (1.6 + 0.08 * mr * nr) + std::max(load, hbm);
         if (us >= best.us) continue;
         const KernelId id8[] = {K_GEMM_DIRECT16, K_GEMM_DIRECT32, K_GEMM_DIRECT64, K_GEMM_DIRECT64};
         const KernelId id4[] = {K_GEMM_W4_DIRECT16, K_GEMM_W4_DIRECT32, K_GEMM_W4_DIRECT64, K_GEMM_W4_DIRECT128};
@@ -298,7 +328,9 @@ DirectPlan plan_direct(const nh_context* ctx, int M, int N, int kt, bool w4) {
 double w4_expanded_us(const nh_context* ctx, size_t m, size_t n, size_t k) {
     const int kt = (int)tiled_k_tiles(k);
     const double expand = 2.0 + (double)n * kt * 96 / 5.7e6;
-    return expand + std::min(tiled_gemm_us(ctx, (int)m, (int)n, kt), plan_direct(ctx, (int)m, (int)n, kt, false).us);
+    double tiled;
+    tiled_gemm_cfg(ctx, (int)m, (int)n, kt, &tiled);
+    return expand + std::min(tiled, plan_direct(ctx, (int)m, (int)n, kt, false).us);
 }
 
 nh_status launch_gemm_direct(nh_context* ctx, const DirectPlan& p, const GemmW8A8Args& g, int w4_zp, float w4_scale,
@@ -336,19 +368,19 @@ nh_status launch_gemm(nh_context* ctx, const int8_t* xq, const float* sx, const 
         const unsigned grid = (unsigned)std::min<int64_t>(tiles, ctx->cu_count);
         return launch(ctx, K_GEMM_P224, grid, 512u, kP224Lds, stream, a, err);
     }
-    // Tile choice, tiled A (tiled_gemm_cfg): M = 128 at 4096 -> 16384 took
-    // 34.4 us on 128 workgroups of 256x128 and 28.5 on 256 of 64x128; M = 256
-    // 41.0 -> 35.0 on 128x128.  Row-major A: 256x128 unless that leaves most
-    // CUs idle, then 128x128.
+    // Tile choice.  Tiled A: by time (tiled_gemm_cfg, plan_direct).  Row-major
+    // A: 256x128 unless that leaves most CUs idle, then 128x128.
     const GemmCfg big = a_tiled ? kTiledCfgs[0] : GemmCfg{K_GEMM_W8A8, 256, 128, 1024, gemm_lds_bytes(256, 128, 3)};
     const GemmCfg small = a_tiled ? kTiledCfgs[1] : GemmCfg{K_GEMM_W8A8_128, 128, 128, 256, gemm_lds_bytes(128, 128, 3)};
     auto tiles = [&](const GemmCfg& c) { return gemm_tiles(c, M, N); };
     const GemmCfg* cfg = nullptr;
     if (a_tiled) {
-        cfg = tiled_gemm_cfg(ctx, M, N);
+        double us;
+        const int at = tiled_gemm_cfg(ctx, M, N, a.kt, &us);
+        if (at >= 0) cfg = &kTiledCfgs[at];
         // the register-direct kernel where it is faster: few or ragged tiles, long K
         const DirectPlan p = plan_direct(ctx, M, N, a.kt, false);
-        if (p.us < tiled_gemm_us(ctx, M, N, a.kt)) return launch_gemm_direct(ctx, p, a, 0, 0.0f, stream, err);
+        if (p.us < us) return launch_gemm_direct(ctx, p, a, 0, 0.0f, stream, err);
     } else if (tiles(big) >= ctx->cu_count / 4 && big.lds <= ctx->max_shared_per_block) {
         cfg = &big;
     } else if (small.lds <= ctx->max_shared_per_block) {

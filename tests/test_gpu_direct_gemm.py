@@ -1,4 +1,4 @@
-"""The register-direct GEMM (gemm_direct.hip) at the edges of its tiles.
+"""The register-direct GEMM (gemm_direct.hip) and the LDS-tiled ones at the edges of their tiles.
 
 Every result is exact (int32 sums, the epilogue's fixed rounding order), so
 outputs equal the exact-integer reference bit for bit, and those of the
@@ -27,7 +27,11 @@ SHAPES = [(1, 16, 16), (17, 1000, 1024), (33, 4099, 208), (64, 130, 4112), (65, 
           (113, 333, 4096), (128, 517, 1040), (129, 1027, 4096), (260, 2690, 1856), (400, 70, 8192), (37, 11008, 4096)]
 
 
-@pytest.mark.parametrize("m,n,k", SHAPES)
+# shapes whose time model takes the LDS tiles (256, 128 and 64 rows), with ragged edges both ways and rows of odd length
+RAGGED = [(1000, 4097, 1024), (2047, 4099, 256), (613, 4099, 2688), (600, 1027, 512), (1025, 8193, 128)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES + RAGGED)
 def test_direct_gemm_bit_exact(ctx, m, n, k):
     print(f"direct gemm m={m} n={n} k={k}", flush=True)
     rng = np.random.default_rng(m * 7 + n)
