@@ -999,15 +999,20 @@ static double expected_experts(size_t experts, size_t routes) {
     return experts * (1.0 - std::pow(1.0 - 1.0 / (double)experts, (double)routes));
 }
 
-// Workgroups per expert: as many as give every CU one at the number of experts
-// that evenly spread routes reach, at least two, and no fewer than 4 N tiles
-// each (8, one per wave, when segments are longer than a 16-row block: every
-// part stages the whole segment).  A CU streams one part's weights at a time,
-// so more parts than CUs cost a second round: 8 tokens over 128 experts top-6
-// (~40 reached) in 2 / 6 / 11 / 16 parts: 55.2 / 32.4 / 36.1 / 42.4 us for
-// the up projection; 16 tokens (~68) in 2 / 3 / 6: 61.4 / 53.1 / 57.8.
+// Workgroups per expert: as many as give every CU one when the routes reach as
+// many experts as evenly spread ones do, plus three standard deviations (their
+// number's variance: E (q - (1 + R / E) q^2), q = e^(-R / E)); at least two, and no
+// fewer than 4 N tiles each (8, one per wave, when segments are longer than a
+// 16-row block: every part stages the whole segment).  A CU streams one part's
+// weights at a time, so a few parts more than CUs cost a second round (8
+// tokens over 128 experts top-6, ~40 reached, in 6 parts: 99 us per layer on
+// some inputs and 120 on others; in 5 parts 99-102), while HBM is busy with
+// 3/4 of the CUs streaming.  The up projection there in 2 / 6 / 11 / 16
+// parts: 55.2 / 32.4 / 36.1 / 42.4 us; 16 tokens in 2 / 3 / 6: 61.4 / 53.1 / 57.8.
 static int expert_parts(const nh_context* ctx, size_t experts, size_t routes, size_t max_rows, size_t n) {
-    const double active = expected_experts(experts, routes);
+    const double mean = expected_experts(experts, routes), load = (double)routes / (double)experts;
+    const double q = std::exp(-load), var = (double)experts * (q - (1.0 + load) * q * q);
+    const double active = std::min((double)experts, mean + 3.0 * std::sqrt(std::max(0.0, var)));
     const int64_t ntiles = (int64_t)((n + 15) / 16), least = max_rows <= 16 ? 4 : 8;
     int64_t parts = (int64_t)(ctx->cu_count / std::max(1.0, active));
     parts = std::min(parts, (ntiles + least - 1) / least);
