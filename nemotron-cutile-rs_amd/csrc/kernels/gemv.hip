@@ -829,6 +829,117 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
     wait_vmcnt_le(0);
 }
 
+// Decode unit for the single row that the fused units do not take: an f32 row
+// (the MLP's intermediate) or one longer than 8192 values, up to kLongChunks
+// 16-byte chunks; one N tile per workgroup.  As there, every workgroup
+// quantizes the row into LDS itself while its first weight tiles are in
+// flight, so the separate quantizer's launch (one workgroup per row) goes; the
+// row comes from L2 once per workgroup.  Each wave then streams its K tiles
+// (wave, wave + 8, ...) through a ring of 16 register sets, one tile reloaded
+// as soon as its MFMA has read it.  Codes, scale and outputs are those of the
+// two launches.  Bound by the weight stream: 1 x 21504 f32 -> 4096 (84 MiB)
+// 22.5 -> 17.1 us, 1 x 12288 bf16 -> 4096 16.4 -> 11.8, 1 x 4096 f32 -> 4096 9.4 ->
+// 7.4.  Two to four rows (their codes one after another in every workgroup)
+// took 20.6 / 25 / 29.1 us at K = 21504 against 22.9-23.4 in two launches.
+template <int DT>
+__device__ __forceinline__ void linear_decode_long(const LinearDecodeArgs& a, int8_t* xs) {
+    constexpr int W = kLongThreads / 64, XR = kLongPerThread;
+    constexpr int VPC = DT == DT_BF16 ? 8 : 4;
+    __shared__ v4i red[W * 64];
+    __shared__ int redi[16];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int N = a.N, K = a.K, kt = a.kt;
+    const int chunks = K / VPC, padded = kt * 64 / VPC;  // codes past K are zeros
+    const int tile = blockIdx.x, n = tile * 16 + (lane & 15);
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(a.x, (uint32_t)K * (DT == DT_BF16 ? 2u : 4u));
+    const __amdgpu_buffer_rsrc_t wr = row_tile_rsrc(a.wq, tile, kt);
+    v4i x[XR], b[kSlab];
+    auto load_tile = [&](int s, int t) { b[s] = buffer_load16_stream(wr, t * 1024 + lane * 16); };
+    // the row first (loads return in issue order), the epilogue's operands,
+    // then the head of the weight stream
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+        const int c = tid + r * kLongThreads;
+        x[r] = buffer_load16(xr, c < chunks ? c * 16 : kOutOfRange);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const float swn = n < N ? a.sw[n] : 0.0f;
+    const float bn = (a.bias && n < N) ? a.bias[n] : 0.0f;
+#pragma unroll
+    for (int s = 0; s < kSlab; ++s) load_tile(s, wave + s * W);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t mb = 0;
+#pragma unroll
+    for (int r = 0; r < XR; ++r) mb = DT == DT_BF16 ? absbits_bf16x8(x[r], mb) : absbits_f32x4(x[r], mb);
+    mb = block_max_u32(DT == DT_BF16 ? absbits_pair_f32(mb) : mb, redi);
+    if (mb >= kInfBits && a.nonfinite && blockIdx.x == 0) {  // the first non-finite value (uniform, rare)
+        int first = 0x7fffffff;
+#pragma unroll
+        for (int r = 0; r < XR; ++r) {
+            const int c = tid + r * kLongThreads;
+            int e = VPC;
+            if constexpr (DT == DT_BF16) {
+                e = bf16x8_first_nonfinite(x[r]);
+            } else {
+#pragma unroll
+                for (int j = VPC - 1; j >= 0; --j)
+                    if (((uint32_t)x[r][j] & 0x7fffffffu) >= kInfBits) e = j;
+            }
+            if (c < chunks && e < VPC) first = min(first, c * VPC + e);
+        }
+        first = block_min_i32(first, redi);
+        if (tid == 0) report_nonfinite(a.nonfinite, a.nonfinite_stage, first, load_as_f32(a.x, first, DT));
+    }
+    const float s = scale_from_amax(f32_from_bits(mb));
+    const float rcp = s > 0.0f ? 1.0f / s : 0.0f;
+    const bool pow2 = scale_is_pow2(s);
+    if (blockIdx.x == 0 && tid == 0 && a.sx_out) a.sx_out[0] = s;
+#pragma unroll
+    for (int r = 0; r < XR; ++r) {
+        const int c = tid + r * kLongThreads;
+        if (c >= padded) break;
+        if constexpr (DT == DT_BF16) {
+            uint32_t code[2];
+            quantize8_bf16(x[r], s, rcp, pow2, code);
+            if (c >= chunks) code[0] = code[1] = 0;
+            *(uint2*)(xs + c * 8) = make_uint2(code[0], code[1]);
+            if (blockIdx.x == 0 && a.xq_out && c < chunks) *(uint2*)(a.xq_out + c * 8) = make_uint2(code[0], code[1]);
+        } else {
+            uint32_t code = quantize4_f32(x[r], s, rcp, pow2);
+            if (c >= chunks) code = 0;
+            *(uint32_t*)(xs + c * 4) = code;
+            if (blockIdx.x == 0 && a.xq_out && c < chunks) *(uint32_t*)(a.xq_out + c * 4) = code;
+        }
+    }
+    lds_publish();  // the codes; the weight tiles stay in flight
+    // every lane reads row 0: the outputs of rows 1..15 are not stored
+    const int8_t* xrow = xs + (lane >> 4) * 16;
+    v4i acc = {0, 0, 0, 0};
+    const int steps = (kt + W - 1) / W;
+    for (int s0 = 0; s0 < steps; s0 += kSlab) {
+#pragma unroll
+        for (int u = 0; u < kSlab; ++u) {
+            const int t = wave + (s0 + u) * W;
+            const v4i xv = *(const v4i*)(xrow + (t < kt ? t : 0) * 64);  // (past kt: the weights are zeros)
+            acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(xv, b[u], acc, 0, 0, 0);
+            load_tile(u, t + kSlab * W);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (reduce_waves(acc, red, W) && n < N && lane < 16)
+        store_y(a.out, a.out_dtype, n, acc[0], s, swn, a.bias, bn, a.relu2);
+}
+
+extern "C" __global__ __launch_bounds__(kLongThreads) void nh_linear_decode_long_kernel(LinearDecodeArgs a) {
+    extern __shared__ __align__(16) int8_t xs[];  // [64 kt] codes
+    if (a.x_dtype == DT_BF16)
+        linear_decode_long<DT_BF16>(a, xs);
+    else
+        linear_decode_long<DT_F32>(a, xs);
+}
+
 extern "C" __global__ __launch_bounds__(512) void nh_linear_decode_w8a8_m1_kernel(LinearDecodeArgs a) {
     extern __shared__ __align__(16) int8_t xs[];  // [W * 1024 + 16] codes
     linear_decode_row<1>(a, xs);

@@ -149,7 +149,15 @@ struct LinearDecodeArgs {
     uint64_t* nonfinite;  // or null: the first non-finite activation (report_nonfinite, nh_device.h)
     uint32_t* row_max;    // or null (streaming unit, f32 out): [gridDim.x][M] largest finite |y| of the
                           // workgroup's outputs per row, as f32 bits (each workgroup writes its own slots)
+    int32_t nonfinite_stage;  // long-row unit: where x stands in its layer
+    int32_t pad_;
 };
+
+// The long-row decode unit (nh_linear_decode_long_kernel): rows of at most
+// kLongChunks 16-byte chunks, kLongThreads threads.
+constexpr int kLongThreads = 512;
+constexpr int kLongPerThread = 11;
+constexpr int kLongChunks = kLongThreads * kLongPerThread;
 
 // G2: W8A32 dequant GEMV; grid = (N tiles, ceil(M / rows per workgroup)).
 struct GemvW8A32Args {

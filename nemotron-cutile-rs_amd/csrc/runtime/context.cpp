@@ -71,6 +71,7 @@ const char* const kKernelSymbols[K_COUNT] = {  // in KernelId order
     "nh_gemm_w4a8_direct32_kernel",      // K_GEMM_W4_DIRECT32
     "nh_gemm_w4a8_direct64_kernel",      // K_GEMM_W4_DIRECT64
     "nh_gemm_w4a8_direct128_kernel",     // K_GEMM_W4_DIRECT128
+    "nh_linear_decode_long_kernel",      // K_LINEAR_DECODE_LONG
 };
 
 void clear_error(nh_error* err) {

@@ -74,6 +74,7 @@ enum KernelId : int {
     K_GEMM_W4_DIRECT32,
     K_GEMM_W4_DIRECT64,
     K_GEMM_W4_DIRECT128,      // up to 64 rows x 128 columns
+    K_LINEAR_DECODE_LONG,     // M = 1, an f32 or long row
     K_COUNT
 };
 
