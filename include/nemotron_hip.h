@@ -192,12 +192,14 @@ nh_status nh_take_nonfinite(nh_context *ctx, uint64_t *nonfinite, nh_stream stre
 /* Quantized linear layer, the drop-in for LinearProjection::project_into
  * with int8 per-row weights (linear.rs:283-342): dynamic per-token
  * quantization of x (f32 or bf16) then G1/G3 + bias.  For bf16 x with
- * k <= 8192 and m <= 4 (m <= 8 when k % 512 == 0) the quantization is fused
- * into the GEMV (one launch; the workspace is not touched); other bf16 x
- * with m <= 16 and k <= 8192 is one launch whose quantizer workgroups hand
- * the codes to its GEMV workgroups through the workspace and a counter slot
- * of the context (kHandoffSlots = 256 slots taken in turn: at most 256 such
- * launches may be in flight at once on one context); otherwise the
+ * k <= 8192 and m <= 4 (m <= 16 when k % 512 == 0 and k <= 4096) the
+ * quantization is fused into the GEMV (one launch; the workspace is not
+ * touched), as it is for most single rows of f32 or of k > 8192 (which still
+ * ask for their workspace); some bf16 x with m <= 16 and 4096 <= k <= 8192 is
+ * one launch whose quantizer workgroups hand the codes to its GEMV workgroups
+ * through the workspace and a counter slot of the context (kHandoffSlots = 256
+ * slots taken in turn: at most 256 such launches may be in flight at once on
+ * one context); otherwise the
  * quantization runs as its own launch into a workspace of
  * nh_linear_w8a8_workspace_size(m, k) bytes, 16-byte aligned (for m <= 16
  * it holds the codes in the GEMV's operand order).  Pass that workspace on
@@ -444,12 +446,14 @@ nh_status nh_tile_weights_int4_host(const uint8_t *packed, size_t packed_len, si
  *  * bf16 x with nh_supports_linear_w4a8(m, n, k) (m <= 16, k <= 8192,
  *    k % 16 == 0): the fused decode unit streams the 4-bit weights once (3..16
  *    rows with k % 512 == 0 and k <= 4096 in one launch, else groups of 4
- *    rows, each streaming them once); workspace may be NULL;
- *  * otherwise (f32 x, prefill-sized m, longer K; k % 16 == 0 and the W8A8
- *    GEMM envelope): the weights are expanded into int8 tiles of code - zp
- *    in the workspace (nh_linear_w4a8_workspace_size(m, n, k) bytes, 16-byte
- *    aligned; LENGTH_MISMATCH "workspace" when smaller) and nh_linear_w8a8's
- *    path runs on them with every row scale equal to `scale`.
+ *    rows, each streaming them once); workspace may be NULL, and with one of
+ *    the size below 5..16 rows of other k read the weights once too;
+ *  * otherwise (f32 x, more rows, longer K; k % 16 == 0 and the W8A8 GEMM
+ *    envelope) a workspace of nh_linear_w4a8_workspace_size(m, n, k) bytes,
+ *    16-byte aligned (LENGTH_MISMATCH "workspace" when smaller): up to a few
+ *    hundred rows a GEMM on the 4-bit weights, for more rows the weights
+ *    expanded into int8 tiles of code - zp there and nh_linear_w8a8's path on
+ *    them with every row scale equal to `scale`.
  * Both are bit-identical to the layer's definition.  Errors in the
  * reference's order: INVALID_SHAPE, INVALID_PARAMS (validate_int4_params,
  * quantize.rs:180-186), INVALID_ROW_COUNT. */

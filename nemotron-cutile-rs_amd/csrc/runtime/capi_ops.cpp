@@ -27,11 +27,11 @@ int gemv_waves(int kt) { return std::max(1, std::min(8, (kt + 15) / 16)); }
 
 // The linear entry point's M ranges: the fused decode unit (quantizer inside
 // the GEMV, one launch) for up to 4 bf16 rows (K <= 8192) and for 3..16 bf16
-// rows (K <= 4096, K % 512 == 0, the streaming form); other bf16 rows up to
-// 16 (K <= 8192) as the handoff launch (quantizer workgroups feeding the
-// tiled-A GEMV's workgroups inside one launch); otherwise quantization into
-// activation tiles + the tiled-A GEMV up to 16 rows (f32 rows, K > 8192),
-// and the MFMA GEMM beyond.
+// rows (K <= 4096, K % 512 == 0, the streaming form), and for one f32 or longer
+// row (long_row_ok); other bf16 rows up to 16 with K = 4096..8192 and few
+// columns as the handoff launch (quantizer workgroups feeding the tiled-A
+// GEMV's workgroups inside one launch); otherwise quantization into
+// activation tiles + the tiled-A GEMV up to 16 rows, and the MFMA GEMMs beyond.
 constexpr size_t kTiledActRows = 16;
 
 // Fused decode unit: kernel, N tiles per workgroup, block size, LDS bytes.
@@ -533,6 +533,36 @@ nh_status linear_w8a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const in
                       uint32_t* row_max = nullptr);
 }  // namespace
 
+namespace {
+
+// nh_linear_w4a8 on the INT4 tiles themselves: the rows' codes as A tiles in the
+// workspace, where the expanded weights would go (in the linear part of it
+// when there are more rows than columns), then the register-direct GEMM.
+// Fits when one of the two holds them: the linear part of 16 rows or fewer is
+// sized for those rows only.
+bool w4_direct_fits(size_t m, size_t n, size_t k) {
+    return tiled_bytes(m, k) <= tiled_bytes(n, k) || m > kTiledActRows;
+}
+
+nh_status linear_w4a8_direct(nh_context* ctx, const DirectPlan& p, const void* x, nh_dtype x_dtype,
+                             const uint8_t* w4_tiled, float scale, uint32_t zero_point, const float* bias, size_t m,
+                             size_t n, size_t k, void* out, nh_dtype out_dtype, void* workspace, uint64_t* nonfinite,
+                             nh_stream stream, nh_error* err) {
+    char* lin = (char*)workspace + align256((size_t)tiled_bytes(n, k)) + align256(n * sizeof(float));
+    const size_t codes = (size_t)tiled_bytes(m, k);
+    const bool in_w8 = codes <= (size_t)tiled_bytes(n, k);
+    int8_t* atiles = (int8_t*)(in_w8 ? workspace : lin);
+    float* sx = (float*)(in_w8 ? lin : lin + align256(codes));
+    nh_status st = launch_quantize(ctx, x, x_dtype, m, k, nullptr, sx, nullptr, atiles, stream, err, 16, nullptr, 1,
+                                   nonfinite, kStageInput);
+    if (st) return st;
+    GemmW8A8Args g{atiles, sx, (const int8_t*)w4_tiled, nullptr, bias, out, (int)m, (int)n, (int)k, 0, 0,
+                   out_dtype, 0, (int)tiled_k_tiles(k), (int)n, 0};
+    return launch_gemm_direct(ctx, p, g, (int)zero_point, scale, stream, err);
+}
+
+}  // namespace
+
 extern "C" {
 
 nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const uint8_t* w4_tiled, float scale,
@@ -561,22 +591,11 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
         float* sw = (float*)(w8 + align256((size_t)tiled_bytes(n, k)));
         void* lin = (char*)sw + align256(n * sizeof(float));
         const size_t lin_bytes = workspace_bytes - (size_t)((char*)lin - (char*)workspace);
-        // up to a few hundred rows: the register-direct GEMM on the INT4 tiles
-        // themselves.  Its A tiles take the place of the expanded weights
-        // (the linear workspace where there are more rows than columns).
+        // up to a few hundred rows: the register-direct GEMM on the INT4 tiles themselves
         const DirectPlan p = plan_direct(ctx, (int)m, (int)n, (int)tiled_k_tiles(k), true);
-        const size_t at_bytes = (size_t)tiled_bytes(m, k);
-        const bool in_w8 = at_bytes <= (size_t)tiled_bytes(n, k);
-        if ((in_w8 || m > kTiledActRows) && p.us < w4_expanded_us(ctx, m, n, k)) {
-            int8_t* atiles = in_w8 ? w8 : (int8_t*)lin;
-            float* sx = in_w8 ? (float*)lin : (float*)((char*)lin + align256(at_bytes));
-            if ((st = launch_quantize(ctx, x, x_dtype, m, k, nullptr, sx, nullptr, atiles, stream, err, 16, nullptr, 1,
-                                      nonfinite, kStageInput)))
-                return st;
-            GemmW8A8Args g{atiles, sx, (const int8_t*)w4_tiled, nullptr, bias, out, (int)m, (int)n, (int)k, 0, 0,
-                           out_dtype, 0, (int)tiled_k_tiles(k), (int)n, 0};
-            return launch_gemm_direct(ctx, p, g, (int)zero_point, scale, stream, err);
-        }
+        if (w4_direct_fits(m, n, k) && p.us < w4_expanded_us(ctx, m, n, k))
+            return linear_w4a8_direct(ctx, p, x, x_dtype, w4_tiled, scale, zero_point, bias, m, n, k, out, out_dtype,
+                                      workspace, nonfinite, stream, err);
         ExpandInt4Args e{w4_tiled, w8, sw, (int64_t)(tiled_int4_bytes(n, k) / 8), (int64_t)n, scale,
                          (int32_t)zero_point};
         if ((st = launch(ctx, K_EXPAND_INT4, grid_for(e.lanes, 256), 256, 0, stream, e, err))) return st;
@@ -609,6 +628,14 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
                              : m <= 8 ? K_LINEAR_DECODE_STREAM_W4_M8
                                       : K_LINEAR_DECODE_STREAM_W4_M16;
         return launch(ctx, kid, grid, 1024u, plan.lds, stream, a, err);
+    }
+    // 5..16 rows otherwise: the register-direct GEMM reads the weights once,
+    // when the caller gave the workspace for the rows' codes (16 x 288 -> 256
+    // 6.9 us against 22.4 in groups, 8 x 8192 -> 4096 12.4 / 23.4)
+    if (m > 4 && workspace && aligned16(workspace) && workspace_bytes >= nh_linear_w4a8_workspace_size(m, n, k)) {
+        if (w4_direct_fits(m, n, k))
+            return linear_w4a8_direct(ctx, plan_direct(ctx, (int)m, (int)n, kt, true), x, x_dtype, w4_tiled, scale,
+                                      zero_point, bias, m, n, k, out, out_dtype, workspace, nonfinite, stream, err);
     }
     // groups of up to 4 rows, each a launch that streams the weights once
     for (size_t r0 = 0; r0 < m; r0 += 4) {
@@ -805,10 +832,17 @@ nh_status linear_w8a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const in
         if (!aligned16(workspace)) return set_error(err, NH_UNSUPPORTED, "workspace must be 16-byte aligned");
         int8_t* tiles = (int8_t*)workspace;
         float* sx = sx_out ? sx_out : (float*)((char*)workspace + align256(act_tiles_bytes(m, k)));
-        if (x_dtype == NH_BF16 && aligned16(x) && k % 8 == 0 && k <= 8192 && ((uintptr_t)xq_out & 7u) == 0) {
-            // one launch: the quantizer workgroups hand the rows to the GEMV
-            // workgroups inside it (M = 8, 8192 -> 4096: 13.57 against 13.96
-            // us in two launches; the 52-layer stack 1.733 against 1.760 ms)
+        // The quantizer's workgroups hand the rows to the GEMV's inside one
+        // launch where that saves more than its wait costs: long rows, and
+        // every workgroup on a CU of its own (8 x 6144 -> 2048 9.9 us against
+        // 10.7 in two launches, 8 x 7680 -> 512 9.0 / 11.4; but 8 x 5120 -> 4096,
+        // 264 workgroups, 12.8 / 10.7, 5 x 2688 -> 4096 11.4 / 8.9, 12 x 688 -> 20115
+        // 23.2 / 9.3), or so much weight per workgroup that a few on shared CUs
+        // do not matter (8 x 8192 -> 4096 13.3 / 13.6, -> 6144 17.2 / 17.8).
+        const size_t tiles_n = (n + 15) / 16, cu = (size_t)ctx->cu_count, ktiles = (size_t)tiled_k_tiles(k);
+        const bool handoff = (ktiles >= 64 && tiles_n + m <= cu) ||
+                             (ktiles >= 128 && tiles_n <= cu * 3 / 2 && m <= 8);
+        if (handoff && x_dtype == NH_BF16 && aligned16(x) && k <= 8192 && ((uintptr_t)xq_out & 7u) == 0) {
             LinearHandoffArgs h{};
             h.q = QuantizeRowsArgs{x, xq_out, sx, nullptr, tiles, (int64_t)m, (int64_t)k, x_dtype, 1, (int)m, 1,
                                    nullptr, nonfinite, nonfinite_stage, 0};
