@@ -105,6 +105,7 @@ nh_status device_error(nh_error* err, hipError_t e, const char* what) {
 
 nh_status bind_device(nh_context* ctx, nh_error* err) {
     if (!ctx) return set_error(err, NH_INVALID_PARAMS, "null context");
+    if (ctx->record) return NH_OK;
     int cur = -1;
     hipError_t e = hipGetDevice(&cur);
     if (e != hipSuccess) return device_error(err, e, "hipGetDevice");
@@ -285,6 +286,38 @@ nh_status nh_stream_synchronize(nh_context* ctx, nh_stream stream, nh_error* err
     hipError_t e = hipStreamSynchronize((hipStream_t)stream);
     if (e != hipSuccess) return device_error(err, e, "hipStreamSynchronize");
     return NH_OK;
+}
+
+nh_context* nh_record_context(int cu_count, size_t lds) {
+    nh_context* ctx = new (std::nothrow) nh_context();
+    if (!ctx) return nullptr;
+    ctx->record = new (std::nothrow) LaunchLog();
+    if (!ctx->record) {
+        delete ctx;
+        return nullptr;
+    }
+    ctx->cu_count = cu_count;
+    ctx->max_shared_per_block = lds;
+    for (int i = 0; i < K_COUNT; ++i) ctx->max_threads[i] = 1024;
+    return ctx;
+}
+
+int nh_record_take(nh_context* ctx, const char** names, uint32_t* gx, uint32_t* gy, int max) {
+    LaunchLog& log = *ctx->record;
+    const int n = log.count;
+    for (int i = 0; i < n && i < max && i < LaunchLog::kMax; ++i) {
+        names[i] = kKernelSymbols[log.launch[i].id];
+        gx[i] = log.launch[i].gx;
+        gy[i] = log.launch[i].gy;
+    }
+    log.count = 0;
+    return n;
+}
+
+void nh_record_free(nh_context* ctx) {
+    if (!ctx) return;
+    delete ctx->record;
+    delete ctx;
 }
 
 // Registry in the spirit of supported_*_kernels(): every device kernel is

@@ -89,6 +89,17 @@ constexpr size_t kScratchBytes = 64ull << 20;
 // kHandoffSlots handoff launches may be in flight at once on one context.
 constexpr uint32_t kHandoffSlots = 256;
 
+// What a recording context (nh_record_context) notes down: the first kMax
+// launches since the last nh_record_take, and how many there were.
+struct LaunchLog {
+    static constexpr int kMax = 64;
+    struct {
+        KernelId id;
+        unsigned gx, gy;
+    } launch[kMax];
+    int count;
+};
+
 }  // namespace nh
 
 struct nh_context {
@@ -106,6 +117,9 @@ struct nh_context {
     // leaves its slot zeroed again.  Calls take the slots in turn.
     uint32_t* handoff;
     std::atomic<uint32_t> handoff_next;
+    // null, except in a recording context: launches are noted here in place
+    // of being made, so the dispatch of the entry points runs without a GPU
+    nh::LaunchLog* record;
 };
 
 namespace nh {
@@ -134,6 +148,12 @@ nh_status launch(nh_context* ctx, KernelId id, unsigned gx, unsigned bx, size_t 
     if (shmem + (size_t)ctx->static_lds[id] > ctx->max_shared_per_block)
         return set_error(err, NH_DEVICE_ERROR, "%s: %zu bytes of LDS requested (%zu available)", kKernelSymbols[id],
                          shmem + (size_t)ctx->static_lds[id], ctx->max_shared_per_block);
+    if (ctx->record) {
+        LaunchLog& log = *ctx->record;
+        if (log.count < LaunchLog::kMax) log.launch[log.count] = {id, gx, gy};
+        ++log.count;
+        return NH_OK;
+    }
     void* params[] = {const_cast<Args*>(&args)};
     hipError_t e = hipModuleLaunchKernel(ctx->fn[id], gx, gy, 1, bx, 1, 1, (unsigned)shmem, (hipStream_t)stream,
                                          params, nullptr);
@@ -145,3 +165,13 @@ inline bool mul_ok(size_t a, size_t b, size_t* out) { return !__builtin_mul_over
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 }  // namespace nh
+
+// Which kernels the entry points launch for a call, for the tests: a context
+// of a device with cu_count CUs and `lds` bytes of LDS per workgroup whose
+// launches are recorded and not made (pointers are only checked for alignment
+// and overlap).  nh_record_take copies up to `max` kernel names, grid widths
+// and heights of the launches since the last call, forgets them and returns
+// their number.  Exported beside the C ABI, no part of it.
+extern "C" nh_context* nh_record_context(int cu_count, size_t lds);
+extern "C" int nh_record_take(nh_context* ctx, const char** names, uint32_t* gx, uint32_t* gy, int max);
+extern "C" void nh_record_free(nh_context* ctx);
