@@ -20,6 +20,11 @@ unsigned grid_for(int64_t items, int per_block) {
     return (unsigned)g;
 }
 
+// Whether [a, a + an) and [b, b + bn) share bytes.
+bool overlap(const void* a, size_t an, const void* b, size_t bn) {
+    return an != 0 && bn != 0 && (uintptr_t)a < (uintptr_t)b + bn && (uintptr_t)b < (uintptr_t)a + an;
+}
+
 // Waves per workgroup of the GEMV family: wave w owns K tiles w, w + W, ...,
 // at most 16 of them per register slab; W = ceil(KT / 16) up to 8 waves
 // (longer K is walked slab by slab).
@@ -110,13 +115,17 @@ bool plan_stream(const nh_context* ctx, size_t m, size_t n, size_t k, DecodePlan
 // threads hold in registers.  Every workgroup quantizes the row, so where
 // the CUs run several of them one after another that must be little next to
 // their weights: K >= 8192 (1 x 12288 bf16 -> 16384 39.2 us against 42.0 in two
-// launches), but 1 x 4096 f32 -> 12288 16.6 against 14.3.
-bool long_row_ok(const nh_context* ctx, const void* x, nh_dtype dtype, size_t m, size_t n, size_t k,
-                 const int8_t* xq_out) {
-    const size_t vpc = dtype == NH_BF16 ? 8 : 4, kt = (size_t)tiled_k_tiles(k);
+// launches), but 1 x 4096 f32 -> 12288 16.6 against 14.3.  They also read it while
+// others already store, so no output may lie over the row (the two launches
+// read it first, and take such calls).
+bool long_row_ok(const nh_context* ctx, const void* x, nh_dtype dtype, size_t m, size_t n, size_t k, const void* out,
+                 nh_dtype out_dtype, const int8_t* xq_out, const float* sx_out) {
+    const size_t vpc = dtype == NH_BF16 ? 8 : 4, kt = (size_t)tiled_k_tiles(k), row = k * (16 / vpc);
     return m == 1 && k % 16 == 0 && aligned16(x) && ((uintptr_t)xq_out & (vpc - 1)) == 0 &&
            kt * 64 / vpc <= (size_t)kLongChunks && ((n + 15) / 16 <= (size_t)ctx->cu_count || kt >= 128) &&
-           kt * 64 + 9 * 1024 <= ctx->max_shared_per_block;
+           kt * 64 + 9 * 1024 <= ctx->max_shared_per_block &&
+           !overlap(x, row, out, n * (out_dtype == NH_BF16 ? 2 : 4)) && !overlap(x, row, xq_out, xq_out ? k : 0) &&
+           !overlap(x, row, sx_out, sx_out ? sizeof(float) : 0);
 }
 
 // Dynamic LDS of the GEMM kernels: a ring of `stages` stages of `ks` K tiles
@@ -865,7 +874,7 @@ nh_status linear_w8a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const in
             h.slot = ctx->handoff + (size_t)(ctx->handoff_next.fetch_add(1) % kHandoffSlots) * 16;
             return launch(ctx, K_LINEAR_HANDOFF, (unsigned)(m + h.consumers), 64u * (g.waves + 1), 0, stream, h, err);
         }
-        if (long_row_ok(ctx, x, x_dtype, m, n, k, xq_out)) {
+        if (long_row_ok(ctx, x, x_dtype, m, n, k, out, out_dtype, xq_out, sx_out)) {
             // one f32 or long row: quantized in the GEMV's workgroups
             LinearDecodeArgs a{};
             a.x = x;

@@ -77,3 +77,29 @@ def test_long_row_still_asks_for_its_workspace(ctx):
     st, err = NH.call_status("nh_linear_w8a8", ctx.handle, d.ptr, NH.F32, d.ptr, d.ptr, None, 1, n, k, d.ptr, NH.F32,
                              None, 0, None, None, None, None)
     assert st == NH.LENGTH_MISMATCH and err.argument == b"workspace"
+
+
+@pytest.mark.parametrize("k", [4096, 21504])
+def test_long_row_overwritten_by_its_own_outputs(ctx, k):
+    """A square f32 layer in place (out = x), and codes written over the row: every value is read before any is written."""
+    print(f"long row in place k={k}", flush=True)
+    n = k if k == 4096 else 512
+    rng = np.random.default_rng(k)
+    x = O.normal_f32(k + 1, k).reshape(1, k)
+    _, xq, sx, _ = O.quantize_rows_f32(x)
+    wq = rng.integers(-127, 128, size=(n, k), dtype=np.int8)
+    sw = rng.uniform(1e-4, 2e-3, n).astype(np.float32)
+    drow, dsw = ctx.upload(wq), ctx.upload(sw)
+    dw = NH.tile_weights(ctx, drow, n, k)
+    ref = linear_w8a8_exact(xq, sx, wq, sw)[0]
+    ws_bytes = NH.lib().nh_linear_w8a8_workspace_size(1, k)
+    ws, out = ctx.empty(ws_bytes, np.uint8), ctx.empty(n, np.float32)
+    for codes in (False, True):
+        dx = ctx.upload(x)
+        NH.call("nh_linear_w8a8", ctx.handle, dx.ptr, NH.F32, dw.ptr, dsw.ptr, None, 1, n, k, out.ptr if codes else dx.ptr,
+                NH.F32, ws.ptr, ws_bytes, dx.ptr if codes else None, None, None, None)
+        ctx.synchronize()
+        got = dx.numpy().reshape(-1)
+        if codes:
+            assert np.array_equal(got.view(np.int8)[:k], xq[0])
+        assert np.array_equal(out.numpy() if codes else got[:n], ref)
