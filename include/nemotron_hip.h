@@ -444,10 +444,10 @@ nh_status nh_tile_weights_int4_host(const uint8_t *packed, size_t packed_len, si
  * exact) on per-token Q2 codes of x, y = ((float)acc * sx) * scale [+ bias].
  * Two device forms:
  *  * bf16 x with nh_supports_linear_w4a8(m, n, k) (m <= 16, k <= 8192,
- *    k % 16 == 0): the fused decode unit streams the 4-bit weights once (3..16
- *    rows with k % 512 == 0 and k <= 4096 in one launch, else groups of 4
- *    rows, each streaming them once); workspace may be NULL, and with one of
- *    the size below 5..16 rows of other k read the weights once too;
+ *    k % 16 == 0): fused decode units, the quantization inside; up to 4 rows,
+ *    up to 16 of k <= 4096 and up to 8 past that are one launch that streams
+ *    the 4-bit weights once, more rows a launch per 8.  The workspace is not
+ *    touched and may be NULL (x not 16-byte aligned: the form below);
  *  * otherwise (f32 x, more rows, longer K; k % 16 == 0 and the W8A8 GEMM
  *    envelope) a workspace of nh_linear_w4a8_workspace_size(m, n, k) bytes,
  *    16-byte aligned (LENGTH_MISMATCH "workspace" when smaller): up to a few

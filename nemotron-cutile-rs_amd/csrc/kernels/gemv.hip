@@ -92,17 +92,16 @@ __device__ __forceinline__ void report_decode_rows(const LinearDecodeArgs& a, co
                          bf16_to_f32(((const uint16_t*)a.x)[first]));
 }
 
-// The same for the wide decode units: xv[j] holds chunk c0 + j stride of
-// the row-major [M][K] input, i.e. the values at flat index 8 chunk + e.
-template <int XR>
-__device__ __forceinline__ void report_decode_chunks(const LinearDecodeArgs& a, const v4i (&xv)[XR], int c0,
-                                                     int stride) {
+// The same for the wide decode units: xv[j] holds chunk chunk_of(j) of the
+// row-major [M][K] input, i.e. the values at flat index 8 chunk + e.
+template <int XR, class ChunkOf>
+__device__ __forceinline__ void report_decode_chunks(const LinearDecodeArgs& a, const v4i (&xv)[XR], ChunkOf chunk_of) {
     __shared__ int red_nf[16];
     int first = 0x7fffffff;
     const int chunks = a.M * (a.K >> 3);
 #pragma unroll
     for (int j = 0; j < XR; ++j) {
-        const int c = c0 + j * stride;
+        const int c = chunk_of(j);
         const int e = bf16x8_first_nonfinite(xv[j]);
         if (c < chunks && e < 8) first = min(first, c * 8 + e);
     }
@@ -527,7 +526,7 @@ __device__ __forceinline__ void linear_decode_wide(const LinearDecodeArgs& a, in
     if (blockIdx.x == 0 && a.nonfinite) {
         bool nonfinite = false;
         for (int r = 0; r < M; ++r) nonfinite |= (uint32_t)rowmax[r] >= 0x7f800000u;
-        if (nonfinite) report_decode_chunks<XR>(a, xv, (int)threadIdx.x, T);
+        if (nonfinite) report_decode_chunks<XR>(a, xv, [&](int j) { return (int)threadIdx.x + j * T; });
     }
     // codes into LDS: chunk c = 8 values of row c / cpr at k = 8 (c % cpr)
 #pragma unroll
@@ -607,7 +606,10 @@ __device__ __forceinline__ void linear_decode_wide(const LinearDecodeArgs& a, in
 // Every load is unconditional (rounds past the run and K tiles past kt read
 // out of range: zeros, no memory traffic), so each wait is a fixed count.
 // Codes and scales are bit-identical to quantize_i8 (quantize8_bf16).
-template <int MM, int XR, int KS, int NB, bool W4 = false>
+// PAD: any K (a multiple of 16): the chunks are dealt as if a row had whole
+// groups of 64, those past K reading zeros, whose codes also fill the row's
+// last K tile (INT4 tiles hold the zero point there, and the row sums do not).
+template <int MM, int XR, int KS, int NB, bool W4 = false, bool PAD = false>
 __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, int8_t* lds) {
     constexpr int NW = 16;
     const int lane = threadIdx.x & 63;
@@ -634,6 +636,34 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
     // 1. activations, epilogue operands, the first PRE rounds of weights
     const __amdgpu_buffer_rsrc_t xrs = make_rsrc(a.x, (uint32_t)M * (uint32_t)K * 2u);
     const int cbase = wave * XR * 64;  // the wave's first chunk
+    // the wave's 64-chunk group j: its row (M: none) and the lane's chunk in it.
+    // PAD deals the groups evenly to the waves (short rows would otherwise all
+    // fall to the first ones).
+    int prow[XR], pk[XR];
+    if constexpr (PAD) {
+        const int gpr = (cpr + 63) >> 6, per = (M * gpr + NW - 1) / NW;
+        int r = wave * per / gpr, q = wave * per - r * gpr;
+#pragma unroll
+        for (int j = 0; j < XR; ++j) {
+            prow[j] = j < per ? min(r, M) : M;
+            pk[j] = q * 64;
+            const int wrap = ++q == gpr;
+            q = wrap ? 0 : q;
+            r += wrap;
+        }
+    }
+    auto row_of = [&](int j) {
+        if constexpr (PAD) return prow[j];
+        else return (cbase + j * 64) / cpr;
+    };
+    auto chunk_of = [&](int j, int row) {
+        if constexpr (PAD) return pk[j] + lane;
+        else return cbase + j * 64 + lane - row * cpr;
+    };
+    auto live = [&](int j) {  // uniform
+        if constexpr (PAD) return prow[j] < M;
+        else return cbase + j * 64 < M * cpr;
+    };
     v4i xv[XR];
     using WB = std::conditional_t<W4, uint2, v4i>;  // one lane's share of a weight tile
     WB b0[KS], b1[KS], b2[KS], b3[KS];
@@ -641,7 +671,12 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
 #pragma unroll
     for (int j = 0; j < XR; ++j) {
         const int c = cbase + j * 64 + lane;
-        xv[j] = buffer_load16(xrs, c < M * cpr ? c * 16 : kOutOfRange);
+        if constexpr (PAD) {
+            const int kc = chunk_of(j, 0);
+            xv[j] = buffer_load16(xrs, live(j) && kc < cpr ? (prow[j] * cpr + kc) * 16 : kOutOfRange);
+        } else {
+            xv[j] = buffer_load16(xrs, c < M * cpr ? c * 16 : kOutOfRange);
+        }
     }
     const uint32_t run_bytes = (uint32_t)min(ntl * 16, N - t0 * 16) * 4u;
     // (W4: one tensor scale, no per-column scales to stage; sw may be null)
@@ -693,12 +728,11 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
     lds_publish();  // rowmax zeroed
     {
         uint32_t m = 0;
-        int cur = cbase / cpr;
+        int cur = row_of(0);
 #pragma unroll
         for (int j = 0; j < XR; ++j) {
-            const int c0 = cbase + j * 64;  // uniform
-            if (c0 < M * cpr) {
-                const int row = c0 / cpr;
+            if (live(j)) {
+                const int row = row_of(j);
                 if (row != cur) {
                     const uint32_t mb = wave_max_dpp_u32(m);
                     if (lane == 0) atomicMax(&rowmax[cur], (int)(mb << 16));
@@ -710,7 +744,7 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
                 m = max(m, bf16x8_absmax_bits(xv[j]));
             }
         }
-        if (cbase < M * cpr) {
+        if (live(0)) {
             const uint32_t mb = wave_max_dpp_u32(m);
             if (lane == 0) atomicMax(&rowmax[cur], (int)(mb << 16));
         }
@@ -726,12 +760,17 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
     if (blockIdx.x == 0 && a.nonfinite) {
         bool nonfinite = false;
         for (int r = 0; r < M; ++r) nonfinite |= (uint32_t)rowmax[r] >= 0x7f800000u;
-        if (nonfinite) report_decode_chunks<XR>(a, xv, cbase + lane, 64);
+        if (nonfinite)
+            report_decode_chunks<XR>(a, xv, [&](int j) {
+                if constexpr (!PAD) return cbase + lane + j * 64;
+                const int kc = chunk_of(j, 0);
+                return live(j) && kc < cpr ? row_of(j) * cpr + kc : 0x7fffffff;
+            });
     }
     // codes into LDS: chunk c = 8 values of row c / cpr at k = 8 (c % cpr);
     // W4: in the nibble order of expand_int4 (act_order_int4), and each row's
     // code sum (zero point, acc - zp * sum_k xq) reduced per row segment
-    int csum = 0, crow = cbase / cpr;
+    int csum = 0, crow = row_of(0);
     auto flush_sum = [&]() {
         int v = csum;
 #pragma unroll
@@ -740,14 +779,13 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
     };
 #pragma unroll
     for (int j = 0; j < XR; ++j) {
-        const int c0 = cbase + j * 64;
-        if (c0 < M * cpr) {
-            const int row = c0 / cpr;
+        if (live(j)) {
+            const int row = row_of(j);
             const float sx = f32_from_bits((uint32_t)__builtin_amdgcn_readlane((int)f32_bits(sx_l), row));
             const float rcp = f32_from_bits((uint32_t)__builtin_amdgcn_readlane((int)f32_bits(rcp_l), row));
             uint32_t code[2];
             quantize8_bf16(xv[j], sx, rcp, scale_is_pow2(sx), code);
-            const int k = (c0 + lane - row * cpr) * 8;
+            const int k = chunk_of(j, row) * 8;
             uint2 st = make_uint2(code[0], code[1]);
             if constexpr (W4) {
                 if (row != crow) {
@@ -759,11 +797,11 @@ __device__ __forceinline__ void linear_decode_stream(const LinearDecodeArgs& a, 
                 csum = __builtin_amdgcn_sdot4((int)code[1], 0x01010101, csum, false);
                 st = act_order_int4(code[0], code[1]);
             }
-            *(uint2*)(xs + (((k >> 6) * 4 + ((k >> 4) & 3)) * MM + row) * 16 + (k & 15)) = st;
-            if (blockIdx.x == 0 && a.xq_out) *(uint2*)(a.xq_out + (int64_t)row * K + k) = make_uint2(code[0], code[1]);
+            if (!PAD || k < kt * 64) *(uint2*)(xs + (((k >> 6) * 4 + ((k >> 4) & 3)) * MM + row) * 16 + (k & 15)) = st;
+            if (blockIdx.x == 0 && a.xq_out && (!PAD || k < K)) *(uint2*)(a.xq_out + (int64_t)row * K + k) = make_uint2(code[0], code[1]);
         }
     }
-    if (W4 && cbase < M * cpr) flush_sum();
+    if (W4 && live(0)) flush_sum();
     if (blockIdx.x == 0 && a.sx_out && tid < M) a.sx_out[tid] = sx_l;
     lds_publish();  // codes and row scales complete
 
@@ -1025,6 +1063,29 @@ extern "C" __global__ __launch_bounds__(1024) void nh_linear_decode_stream_w4_m8
 extern "C" __global__ __launch_bounds__(1024) void nh_linear_decode_stream_w4_m16_kernel(LinearDecodeArgs a) {
     extern __shared__ __align__(16) int8_t lds[];
     linear_decode_stream<16, 8, 4, 2, true>(a, lds);
+}
+
+// 5..16 rows of the other K on INT4 tiles: up to 4096 in one launch, past
+// that 8 rows at a time with 8 K tiles per wave (the codes of 16 would not fit
+// the LDS).  Bound by the quantization in every workgroup ahead of few rounds
+// of weights.  Against groups of 4 rows, each streaming the weights: 5 x 288 ->
+// 256 5.8 against 8.4 us, 16 x 2704 -> 4096 11.9 / 33.8, 8 x 8192 -> 4096 15.7 /
+// 24.2, 16 x 8192 -> 4096 31.4 / 48.1.  (A quantizer launch into the caller's
+// workspace and the register-direct GEMM take 5.9 / 9.2 / 12.4 / 13.4, but
+// these shapes run without one.)
+extern "C" __global__ __launch_bounds__(1024) void nh_linear_decode_stream_w4_any_m8_kernel(LinearDecodeArgs a) {
+    extern __shared__ __align__(16) int8_t lds[];
+    linear_decode_stream<8, 4, 4, 2, true, true>(a, lds);
+}
+
+extern "C" __global__ __launch_bounds__(1024) void nh_linear_decode_stream_w4_any_m16_kernel(LinearDecodeArgs a) {
+    extern __shared__ __align__(16) int8_t lds[];
+    linear_decode_stream<16, 8, 4, 2, true, true>(a, lds);
+}
+
+extern "C" __global__ __launch_bounds__(1024) void nh_linear_decode_stream_w4_long_m8_kernel(LinearDecodeArgs a) {
+    extern __shared__ __align__(16) int8_t lds[];
+    linear_decode_stream<8, 8, 8, 2, true, true>(a, lds);
 }
 
 // G2: W8A32 dequant GEMV, y[m][n] = sum_k x[m][k] * q[n][k] * s[n].  The

@@ -95,20 +95,35 @@ bool plan_decode(const nh_context* ctx, size_t m, size_t n, size_t k, DecodePlan
 // number of rounds, as few workgroups as that many rounds need.  (At K = 8192
 // each CU would load 128 KiB of activations, as much as its share of a
 // 4096-wide output's weights: 16.4 us against 14.7 in two launches.)
-bool plan_stream(const nh_context* ctx, size_t m, size_t n, size_t k, DecodePlan* p, unsigned* grid) {
-    if (m < 3 || m > 16 || k % 512 != 0 || k > 4096) return false;
-    const size_t mm = m <= 4 ? 4 : m <= 8 ? 8 : 16;
+bool plan_stream_grid(const nh_context* ctx, KernelId kid, size_t mm, size_t n, size_t k, DecodePlan* p, unsigned* grid) {
     const size_t tiles = (n + 15) / 16, cu = (size_t)ctx->cu_count;
     const size_t rounds = (tiles + cu - 1) / cu;
     if (rounds > 64) return false;  // a run's scales and bias: at most 1024 LDS floats each
     // codes [KT][4][MM][16], two sets of 16 partial tiles, the run's scales
     // and bias, row maxima, row scales and (W4) row code sums
-    const size_t lds = (k / 64) * 64 * mm + 2 * 16 * 64 * 16 + 2 * 1024 * 4 + 3 * mm * 4;
+    const size_t lds = (size_t)tiled_k_tiles(k) * 64 * mm + 2 * 16 * 64 * 16 + 2 * 1024 * 4 + 3 * mm * 4;
     if (lds > ctx->max_shared_per_block) return false;
-    *p = DecodePlan{mm == 4 ? K_LINEAR_DECODE_STREAM_M4 : mm == 8 ? K_LINEAR_DECODE_STREAM_M8 : K_LINEAR_DECODE_STREAM_M16,
-                    0, 1024, lds};
+    *p = DecodePlan{kid, 0, 1024, lds};
     *grid = (unsigned)((tiles + rounds - 1) / rounds);
     return true;
+}
+
+bool plan_stream(const nh_context* ctx, size_t m, size_t n, size_t k, DecodePlan* p, unsigned* grid) {
+    if (m < 3 || m > 16 || k % 512 != 0 || k > 4096) return false;
+    const size_t mm = m <= 4 ? 4 : m <= 8 ? 8 : 16;
+    const KernelId kid =
+        mm == 4 ? K_LINEAR_DECODE_STREAM_M4 : mm == 8 ? K_LINEAR_DECODE_STREAM_M8 : K_LINEAR_DECODE_STREAM_M16;
+    return plan_stream_grid(ctx, kid, mm, n, k, p, grid);
+}
+
+// The INT4 form of 5..16 rows for the other K (multiples of 16): up to 4096,
+// and up to 8 rows past that.
+bool plan_stream_w4_any(const nh_context* ctx, size_t m, size_t n, size_t k, DecodePlan* p, unsigned* grid) {
+    if (m > (k <= 4096 ? 16u : 8u) || k > 8192) return false;
+    const KernelId kid = k > 4096 ? K_LINEAR_DECODE_STREAM_W4_LONG_M8
+                         : m <= 8 ? K_LINEAR_DECODE_STREAM_W4_ANY_M8
+                                  : K_LINEAR_DECODE_STREAM_W4_ANY_M16;
+    return plan_stream_grid(ctx, kid, m <= 8 ? 8 : 16, n, k, p, grid);
 }
 
 // The long-row decode unit takes one row of whole 16-byte chunks that its 512
@@ -546,13 +561,8 @@ namespace {
 
 // nh_linear_w4a8 on the INT4 tiles themselves: the rows' codes as A tiles in the
 // workspace, where the expanded weights would go (in the linear part of it
-// when there are more rows than columns), then the register-direct GEMM.
-// Fits when one of the two holds them: the linear part of 16 rows or fewer is
-// sized for those rows only.
-bool w4_direct_fits(size_t m, size_t n, size_t k) {
-    return tiled_bytes(m, k) <= tiled_bytes(n, k) || m > kTiledActRows;
-}
-
+// when there are more row tiles than column tiles; that part holds A tiles
+// then, as 16 rows or fewer are one row tile), then the register-direct GEMM.
 nh_status linear_w4a8_direct(nh_context* ctx, const DirectPlan& p, const void* x, nh_dtype x_dtype,
                              const uint8_t* w4_tiled, float scale, uint32_t zero_point, const float* bias, size_t m,
                              size_t n, size_t k, void* out, nh_dtype out_dtype, void* workspace, uint64_t* nonfinite,
@@ -602,7 +612,7 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
         const size_t lin_bytes = workspace_bytes - (size_t)((char*)lin - (char*)workspace);
         // up to a few hundred rows: the register-direct GEMM on the INT4 tiles themselves
         const DirectPlan p = plan_direct(ctx, (int)m, (int)n, (int)tiled_k_tiles(k), true);
-        if (w4_direct_fits(m, n, k) && p.us < w4_expanded_us(ctx, m, n, k))
+        if (p.us < w4_expanded_us(ctx, m, n, k))
             return linear_w4a8_direct(ctx, p, x, x_dtype, w4_tiled, scale, zero_point, bias, m, n, k, out, out_dtype,
                                       workspace, nonfinite, stream, err);
         ExpandInt4Args e{w4_tiled, w8, sw, (int64_t)(tiled_int4_bytes(n, k) / 8), (int64_t)n, scale,
@@ -638,17 +648,13 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
                                       : K_LINEAR_DECODE_STREAM_W4_M16;
         return launch(ctx, kid, grid, 1024u, plan.lds, stream, a, err);
     }
-    // 5..16 rows otherwise: the register-direct GEMM reads the weights once,
-    // when the caller gave the workspace for the rows' codes (16 x 288 -> 256
-    // 6.9 us against 22.4 in groups, 8 x 8192 -> 4096 12.4 / 23.4)
-    if (m > 4 && workspace && aligned16(workspace) && workspace_bytes >= nh_linear_w4a8_workspace_size(m, n, k)) {
-        if (w4_direct_fits(m, n, k))
-            return linear_w4a8_direct(ctx, plan_direct(ctx, (int)m, (int)n, kt, true), x, x_dtype, w4_tiled, scale,
-                                      zero_point, bias, m, n, k, out, out_dtype, workspace, nonfinite, stream, err);
-    }
-    // groups of up to 4 rows, each a launch that streams the weights once
-    for (size_t r0 = 0; r0 < m; r0 += 4) {
-        const size_t rows = std::min<size_t>(4, m - r0);
+    // otherwise launches over groups of rows, each streaming the weights once:
+    // all of 5..16 rows of K <= 4096, 5..8 past that, and groups of up to 4 by the
+    // one-tile units.  No workspace: a call may share its buffer with others.
+    for (size_t r0 = 0, rows; r0 < m; r0 += rows) {
+        rows = std::min<size_t>(k <= 4096 ? 16 : 8, m - r0);
+        const bool wide = rows > 4 && plan_stream_w4_any(ctx, rows, n, k, &plan, &grid);
+        if (!wide) rows = std::min<size_t>(4, rows);
         const size_t mm = rows == 1 ? 1 : rows <= 2 ? 2 : 4;
         const KernelId kid = mm == 1 ? K_LINEAR_DECODE_W4_M1 : mm == 2 ? K_LINEAR_DECODE_W4_ROW2 : K_LINEAR_DECODE_W4_ROW4;
         LinearDecodeArgs a{};
@@ -668,6 +674,11 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
         a.w4_scale = scale;
         a.row0 = (int)r0;  // the group's first row: non-finite inputs are indexed in the whole x
         a.nonfinite = nonfinite;
+        if (wide) {
+            a.waves = 16;
+            if ((st = launch(ctx, plan.kid, grid, 1024u, plan.lds, stream, a, err))) return st;
+            continue;
+        }
         const size_t lds = mm * ((size_t)w * 1024 + 16);
         if (lds > ctx->max_shared_per_block) return set_error(err, NH_UNSUPPORTED, "LDS too small");
         if ((st = launch(ctx, kid, (unsigned)((n + 15) / 16), (unsigned)(64 * w), lds, stream, a, err))) return st;

@@ -72,6 +72,9 @@ const char* const kKernelSymbols[K_COUNT] = {  // in KernelId order
     "nh_gemm_w4a8_direct64_kernel",      // K_GEMM_W4_DIRECT64
     "nh_gemm_w4a8_direct128_kernel",     // K_GEMM_W4_DIRECT128
     "nh_linear_decode_long_kernel",      // K_LINEAR_DECODE_LONG
+    "nh_linear_decode_stream_w4_any_m8_kernel",   // K_LINEAR_DECODE_STREAM_W4_ANY_M8
+    "nh_linear_decode_stream_w4_any_m16_kernel",  // K_LINEAR_DECODE_STREAM_W4_ANY_M16
+    "nh_linear_decode_stream_w4_long_m8_kernel",  // K_LINEAR_DECODE_STREAM_W4_LONG_M8
 };
 
 void clear_error(nh_error* err) {

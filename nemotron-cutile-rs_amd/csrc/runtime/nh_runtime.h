@@ -75,6 +75,9 @@ enum KernelId : int {
     K_GEMM_W4_DIRECT64,
     K_GEMM_W4_DIRECT128,      // up to 64 rows x 128 columns
     K_LINEAR_DECODE_LONG,     // M = 1, an f32 or long row
+    K_LINEAR_DECODE_STREAM_W4_ANY_M8,   // M <= 8, K <= 4096 of any multiple of 16, INT4 weights
+    K_LINEAR_DECODE_STREAM_W4_ANY_M16,  // M <= 16
+    K_LINEAR_DECODE_STREAM_W4_LONG_M8,  // M <= 8, K <= 8192
     K_COUNT
 };
 

@@ -39,3 +39,15 @@ def test_single_row_under_its_own_outputs_takes_two_launches(rec, x_dtype, k):
     assert rec.linear(1, n, k, x_dtype, xq_out=X + row) == ["linear_decode_long"]
     assert rec.linear(1, n, k, x_dtype, sx_out=X + row - 4) == two
     assert rec.linear(1, n, k, x_dtype, sx_out=X + row) == ["linear_decode_long"]
+
+
+# W4A8 decode never writes the workspace, given or not: a buffer that calls on several streams share is not raced on.
+@pytest.mark.parametrize("m", range(1, 17))
+@pytest.mark.parametrize("k", [16, 288, 512, 1040, 4080, 4096, 4112, 5120, 8176, 8192])
+def test_w4a8_decode_ignores_its_workspace(rec, m, k):
+    for n in (5, 256, 4096, 300000):
+        given, none = rec.w4a8(m, n, k), rec.w4a8(m, n, k, workspace=False)
+        assert given == none and all(name.startswith("linear_decode") for name in given)
+        # and the weights are streamed once, or once per 8 rows of K > 4096, where a workgroup's run of tiles fits
+        if m > 2 and n < 262144:
+            assert len(given) <= (1 if k <= 4096 else (m + 7) // 8)
