@@ -1142,11 +1142,22 @@ static nh_status launch_expert_gemm(nh_context* ctx, KernelId id, ExpertGemmArgs
     e.streams = kExpertWaves;
     e.tiles_per_wg = tiles_per_wg;
     e.row_blocks = row_blocks;
-    // the search for the experts with routes only where many have none (512
-    // tokens over 128 experts, where it finds the same order: 0.5 us per launch)
-    e.compact = expected_experts(experts, routes) < 0.9 * (double)experts;
+    // Packed onto the experts with routes (a search of 0.2-0.9 us per launch)
+    // where their workgroups then fit one round of CUs and would not in natural
+    // order: more slots than CUs, and so many of them live that some CUs would
+    // get two (half the CUs' worth, or one of 4 slots per CU and up); or, past
+    // one round, where three of four experts have no route.  Natural order /
+    // packed, us: 128 experts of 1168 x 688 with 16 routes 48.7 / 36.5 per
+    // layer, 64 of 1312 x 2560 with 14 71.1 / 53.8, 253 of 272 x 2192 with 112
+    // 20.1 / 13.3; but 16 of 1024 x 512 with 12 31.1 / 31.5, 197 of 240 x 368
+    // with 216 (262 workgroups packed) 9.9 / 11.6, 1024 of 192 x 1408 with 620
+    // 62.1 / 70.2.
+    const double cu = ctx->cu_count, live = expected_experts(experts, routes), all = (double)parts * (double)experts;
+    const double packed = parts * live;
+    e.compact = all > cu && (packed <= cu ? 2 * packed >= cu || all > 4 * cu
+                                          : (double)experts >= 4 * live && packed <= 4 * cu);
     const size_t slots = e.compact ? std::min(experts, routes) : experts;
-    return launch(ctx, id, (unsigned)(parts * slots), (unsigned)(64 * kExpertWaves), lds, stream, e, err);
+    return launch(ctx, id, (unsigned)parts, (unsigned)(64 * kExpertWaves), lds, stream, e, err, (unsigned)slots);
 }
 
 // Whether the MoE layer's two projections run as the fused expert-block

@@ -51,3 +51,15 @@ def test_w4a8_decode_ignores_its_workspace(rec, m, k):
         # and the weights are streamed once, or once per 8 rows of K > 4096, where a workgroup's run of tiles fits
         if m > 2 and n < 262144:
             assert len(given) <= (1 if k <= 4096 else (m + 7) // 8)
+
+
+# MoE experts: a slot per (expert, part); fewer slots than experts where the workgroups search for the experts with routes.
+# Not where all slots have a CU, the live ones are few, or the packed ones more than a round (of few empty experts).
+@pytest.mark.parametrize("experts,routes,parts,slots", [(16, 12, 8, 16), (136, 1, 8, 1), (30, 1, 8, 30), (128, 126, 2, 128),
+                                                        (128, 48, 4, 48), (128, 3072, 2, 128), (184, 125, 2, 125),
+                                                        (512, 300, 2, 512), (1024, 48, 4, 48), (1024, 180, 2, 180),
+                                                        (1024, 1428, 2, 1024)])
+def test_expert_slots(rec, experts, routes, parts, slots):
+    (name, gx, gy), = rec.launches("nh_moe_grouped_gemm_w8a8", 1 << 40, 2 << 40, 0, 1, 3 << 40, 4 << 40, routes, routes, experts,
+                                   5 << 40, 6 << 40, 512, 1024, 0, 7 << 40, None)
+    assert (name, gx, gy) == ("moe_expert_gemm", parts, slots)
