@@ -56,10 +56,7 @@ template <int MR, int NR, bool W4, bool ST>
 __device__ __forceinline__ void direct_tile(const GemmDirectArgs& d, int8_t* lds, int mt0, int nt0) {
     constexpr int W = kDirectWaves, F = MR * NR;
     constexpr int kTile = W4 ? 512 : 1024;
-    // K tiles in flight per wave: what fits 256 registers next to the accumulators
-    constexpr int kSlot = 4 * MR + (W4 ? 2 : 4) * NR;
-    constexpr int kFit = (216 - 4 * F - (W4 ? MR : 0)) / kSlot;
-    constexpr int D = kFit < 2 ? 2 : kFit > 4 ? 4 : kFit;
+    constexpr int D = direct_depth(MR, NR, W4);  // K tiles in flight per wave
     const GemmW8A8Args& a = d.g;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

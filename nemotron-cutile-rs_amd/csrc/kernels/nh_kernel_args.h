@@ -228,7 +228,14 @@ struct GemmW8A8Args {
     int32_t pad_;
 };
 
-// G3 with both operands loaded straight into registers (gemm_direct.hip).
+// G3 with both operands loaded straight into registers (gemm_direct.hip): K
+// tiles in flight per wave of a tile of mr x nr fragments, what fits 256
+// registers next to the accumulators.
+constexpr int direct_depth(int mr, int nr, bool w4) {
+    const int fit = (216 - 4 * mr * nr - (w4 ? mr : 0)) / (4 * mr + (w4 ? 2 : 4) * nr);
+    return fit < 2 ? 2 : fit > 4 ? 4 : fit;
+}
+
 struct GemmDirectArgs {
     GemmW8A8Args g;     // xq: tiled A; wq: tiled int8 [N][K], or tiled INT4 (then sw is unused)
     int32_t groups;     // row groups: group q owns M tiles [q T / groups, (q + 1) T / groups), T = ceil(M / 16)

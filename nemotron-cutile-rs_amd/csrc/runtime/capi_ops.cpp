@@ -237,28 +237,17 @@ nh_status launch_gemv(nh_context* ctx, const int8_t* xq, const float* sx, const 
                   a, err);
 }
 
-// The persistent 256 x 224 GEMM (gemm_persistent.hip) when its contract
-// holds and its tiles fill rounds of CUs with less work per CU than the
-// loader-wave kernel's 256 x 128 tiles: rounds x tile area (the 21504-wide
-// up projection at M = 2048: 3 rounds of 256 x 224 against 5.5 of 256 x 128;
-// measured 201-203 against 231-236 us).
+// The persistent 256 x 224 GEMM (gemm_persistent.hip): whether its contract holds.
 // Its LDS: two A slots of 2 x 16 tiles, three B slots of 2 x 14 tiles (the
 // weights run a stage further ahead), three scale buffers, a spare KiB.
 constexpr size_t kP224Lds = 2 * 8 * ((2 * 256 / 16 + 7) / 8) * 1024 + 3 * (2 * 224 / 16) * 1024 + 3 * 3 * 1024 + 1024;
 
-bool use_persistent_224(const nh_context* ctx, const void* xq, const float* sx, const float* sw, const float* bias,
-                        int M, int N, int kt, const void* out, nh_dtype out_dtype) {
+bool persistent_224_ok(const nh_context* ctx, const void* xq, const float* sx, const float* sw, const float* bias,
+                       int M, int N, int kt, const void* out, nh_dtype out_dtype) {
     const size_t esz = out_dtype == NH_BF16 ? 2 : 4;
-    if (kt % 2 != 0 || M % 4 != 0 || N % 4 != 0 || !aligned16(xq) || !aligned16(sx) || !aligned16(sw) ||
-        !aligned16(bias) || !aligned16(out) || (uint64_t)M * N * esz >= (1ull << 31) ||
-        kP224Lds > ctx->max_shared_per_block)
-        return false;
-    const int64_t cu = ctx->cu_count, tm = (M + 255) / 256;
-    const int64_t tiles_p = tm * ((N + 223) / 224), tiles_o = tm * ((N + 127) / 128);
-    const int64_t work_p = (tiles_p + cu - 1) / cu * 224, work_o = (tiles_o + cu - 1) / cu * 128;
-    // (one round on at least half of the CUs: 500 x 21504 x 4096, 192 tiles,
-    // 55.9 us against 61.6 for 256 + 160 smaller ones; 768 x 16384 x 4096 60.7 / 78.3)
-    return 2 * tiles_p >= cu && work_p < work_o;
+    return kt % 2 == 0 && M % 4 == 0 && N % 4 == 0 && aligned16(xq) && aligned16(sx) && aligned16(sw) &&
+           aligned16(bias) && aligned16(out) && (uint64_t)M * N * esz < (1ull << 31) &&
+           kP224Lds <= ctx->max_shared_per_block;
 }
 
 // The LDS-tiled G3 kernels (gemm.hip) on tiled A, largest first.
@@ -277,44 +266,49 @@ int64_t gemm_tiles(const GemmCfg& c, int M, int N) {
     return (int64_t)((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
 }
 
-// Time in us of tile choice `at` on cold weights: a launch, and per round of
-// workgroups an epilogue and what the kernel's stage loop takes per 64-deep K
-// tile, more with more of the CUs busy (their clock, and the weight stream).
-// The larger tiles have a CU to themselves, so their rounds are whole (256 x
-// 128: a last round at most half full runs as 128 x 128 tiles); two or three of
-// the smaller ones share one.  Fitted to 342 shapes of 17..2048 rows, 1024..
-// 16384 columns and K = 1024..8192 (each to 7-12% r.m.s.).
-double tiled_gemm_us(const nh_context* ctx, int at, int M, int N, int kt) {
-    const int64_t t = gemm_tiles(kTiledCfgs[at], M, N), cu = ctx->cu_count;
-    const double whole = (double)((t + cu - 1) / cu), avg = std::max(1.0, (double)t / cu);
-    const double fill = std::min(1.0, (double)t / cu);
-    switch (at) {
-    case 0: {
-        const double rounds = t > cu && t % cu != 0 && t % cu <= cu / 2 ? (double)(t / cu) + 0.62 : whole;
-        return -0.35 + rounds * (8.35 + kt * (0.251 + 0.167 * fill));
-    }
-    case 1: return 1.63 + whole * (3.96 + kt * (0.197 + 0.064 * fill));
-    case 2: return 3.32 + 1.17 * avg + kt * (0.031 * avg + whole * (0.144 + 0.013 * fill));
-    default: return 3.79 + kt * (0.042 * avg + whole * (0.147 - 0.047 * fill));
-    }
+// What a GEMM on tiled A takes, in us: the kernels' choice is the least of
+// these.  Coefficients fitted to the choice on 1600 shapes of 17..2048 rows,
+// 64..131072 columns and K = 64..21504 with weights not in any cache, and 600
+// with one matrix called over and over, each timed with all eight kernels (the
+// times: profiles/gemm_choice.csv).  Over them and over 800 others the choice
+// is within 1% of the best on average (2% in cache); a model of the LDS tiles
+// alone, fitted from K = 1024 on, with the persistent kernel ahead of it, was
+// 7% off, and up to 2.9 times (24 x 38400 x 80 13.9 us on the persistent kernel,
+// 4.8 on 64 x 64 tiles; 64 x 33280 x 3440 43 / 23).
+//
+// A tile kernel: a launch; per whole round of workgroups an epilogue and what
+// its stage loop takes per 64-deep K tile whatever the tile holds, more with
+// more CUs busy (their clock) and with weights that come from HBM (`cold`,
+// from 4 MB on); for each workgroup that shares a CU its own MFMAs.  Beside
+// that runs the memory traffic, weights and outputs (f32 ones as much as 1 +
+// out_f32 bf16 ones); the two overlap in part (root of the squares).
+struct TileTime {
+    double launch, round, kt, kt_fill, kt_cold, kt_each, hbm, out, out_f32;
+};
+constexpr TileTime kTileTime[] = {{1.90, 5.69, 0.148, 0.074, 0.034, 0.106, 9.0, 3.23, 0.19},  // kTiledCfgs[0..3]
+                                  {3.02, 1.93, 0.151, 0.086, 0.041, 0.003, 7.9, 1.65, 0.24},
+                                  {2.50, 1.53, 0.162, 0.018, 0.019, 0.000, 6.1, 4.39, 0.48},
+                                  {2.95, 0.18, 0.082, -0.001, 0.003, 0.101, 9.0, 2.11, 0.12}};
+constexpr TileTime kP224Time = {3.84, 6.34, 0.547, 0.022, 0.085, 0.0, 8.9, 2.58, 0.0};
+
+// A GEMM's sizes as the models use them.
+struct GemmSize {
+    int M, N, kt;
+    double weights, outputs;  // MB (outputs as bf16)
+    bool f32_out;
+};
+
+GemmSize gemm_size(int M, int N, int kt, nh_dtype out_dtype) {
+    return GemmSize{M, N, kt, (double)N * kt * 64e-6, (double)M * N * 2e-6, out_dtype == NH_F32};
 }
 
-// The fastest of them by that model, and its time; -1 when the LDS holds none.
-// (The largest tile that fills every CU, which the choice once was, is far off
-// where its tiles leave a second round nearly empty: 1024 x 4099 x 2688 on 264
-// tiles of 128 x 128 32.0 us, on 132 of 256 x 128 24.9; 613 x 10304 x 2688 36.7 / 28.3.)
-int tiled_gemm_cfg(const nh_context* ctx, int M, int N, int kt, double* us) {
-    int best = -1;
-    *us = 1e30;
-    for (int at = 0; at < 4; ++at) {
-        if (kTiledCfgs[at].lds > ctx->max_shared_per_block) continue;
-        const double u = tiled_gemm_us(ctx, at, M, N, kt);
-        if (best < 0 || u < *us) {
-            best = at;
-            *us = u;
-        }
-    }
-    return best;
+double tile_us(const nh_context* ctx, const TileTime& c, int bm, int bn, const GemmSize& g) {
+    const double cu = ctx->cu_count, t = (double)((g.M + bm - 1) / bm) * (double)((g.N + (int64_t)bn - 1) / bn);
+    const double rounds = std::ceil(t / cu), each = std::max(1.0, t / cu), fill = std::min(1.0, t / cu);
+    const double loop = rounds * (c.round + g.kt * (c.kt + c.kt_fill * fill + c.kt_cold * std::min(1.0, g.weights / 4))) +
+                        each * g.kt * c.kt_each;
+    const double mem = g.weights / c.hbm + g.outputs * (g.f32_out ? 1 + c.out_f32 : 1.0) / c.out;
+    return c.launch + std::sqrt(loop * loop + mem * mem);
 }
 
 // The register-direct GEMM (gemm_direct.hip): its tile for a shape, and the
@@ -326,31 +320,50 @@ struct DirectPlan {
     double us;
 };
 
-// Fitted to the same shapes: a launch, then per round of workgroups an epilogue, and
-// per K tile the fragments through the CU's load path (80 KiB per us), or the
-// weights from HBM (5.6 TB/s) where that is longer.  Against the LDS tiles
-// (tiled_gemm_cfg), both sides measured at M x N x K: 17 x 2688 x 2688 5.5 / 11.8
-// us, 77 x 6144 x 4096 11.5 / 15.8, 400 x 2688 x 4096 15.5 / 20.9, 64 x 16384 x
-// 1024 7.8 / 6.8, 512 x 16384 x 4096 49.2 / 36.2.
-DirectPlan plan_direct(const nh_context* ctx, int M, int N, int kt, bool w4) {
+// Its model: a launch, more with more CUs taking part; per round (or partly,
+// INT4, per CU's share of one: two workgroups of a CU overlap there) an
+// epilogue per fragment, and per K tile the fragments through the CU's load
+// path (`a` and `b` us per KiB: 80 KiB per us), also, at `ahead` of the cost,
+// for the loads past the end that a wave's `depth` K tiles in flight round up
+// to; beside that the memory traffic and a wave's chain of dependent
+// steps.  Against the LDS tiles, both measured at M x N x K: 17 x 2688 x 2688
+// 5.5 / 11.8 us, 77 x 6144 x 4096 11.5 / 15.8, 400 x 2688 x 4096 15.5 / 20.9, 64 x
+// 16384 x 1024 7.8 / 6.8, 512 x 16384 x 4096 49.2 / 36.2.
+struct DirectTime {
+    double whole, a, b, launch, round, frag, hbm, out, fill, out_f32, ahead, step;
+};
+constexpr DirectTime kDirectTime = {1.00, 0.0108, 0.0145, 2.50, 0.02, 0.042, 6.8, 1.81, 0.0, 0.33, 0.89, 0.78};
+constexpr DirectTime kDirectTimeW4 = {0.83, 0.0131, 0.0288, 3.65, 0.36, 0.093, 8.9, 20.0, 0.0, 1.0, 0.68, 0.52};
+
+// partial fragments of 4 waves, row and column scales, bias, INT4 row sums
+constexpr size_t kDirectLds = 4 * 16 * 1024 + 3 * 128 * 4 + 4 * 128 * 4;
+constexpr double kNoPlan = 1e30;
+
+DirectPlan plan_direct(const nh_context* ctx, const GemmSize& g, bool w4) {
     DirectPlan best{};
-    best.us = 1e30;
-    const int mtiles = (M + 15) / 16;
+    best.us = kNoPlan;
+    if (kDirectLds > ctx->max_shared_per_block) return best;
+    const DirectTime& c = w4 ? kDirectTimeW4 : kDirectTime;
+    const int mtiles = (g.M + 15) / 16, steps = (g.kt + 3) / 4;
     const double cu = ctx->cu_count;
+    const double mem = g.weights * (w4 ? 0.5 : 1.0) / c.hbm + g.outputs * (g.f32_out ? 1 + c.out_f32 : 1.0) / c.out;
     for (int nr : {1, 2, 4, 8}) {
         if (nr == 8 && !w4) break;
         const int maxr = nr == 8 ? 4 : 8;
         const int groups = (mtiles + maxr - 1) / maxr;
         const int mr = (mtiles + groups - 1) / groups;
-        const int64_t tn = (N + 16 * nr - 1) / (16 * nr), wgs = tn * groups;
+        const int64_t tn = ((int64_t)g.N + 16 * nr - 1) / (16 * nr), wgs = tn * groups;
         if ((tn + 7) / 8 * 8 * groups > kMaxGrid) continue;
-        // between whole rounds (a CU with two workgroups shares its load path)
-        // and the average
-        const double rounds = 0.5 * std::ceil((double)wgs / cu) + 0.5 * std::max(1.0, (double)wgs / cu);
-        const double load = rounds * kt * (mr + (w4 ? 0.5 : 1.0) * nr) / 80.0 *
-                            (0.85 + 0.2 * std::min(1.0, (double)wgs / cu));
-        const double hbm = (double)N * kt * (w4 ? 32 : 64) / 5.6e6;
-        const double us = 2.0 + rounds * (1.6 + 0.08 * mr * nr) + std::max(load, hbm);
+        const double share = (double)wgs / cu;
+        const double rounds = c.whole * std::ceil(share) + (1 - c.whole) * std::max(1.0, share);
+        const int depth = direct_depth(mr, nr, w4);
+        const int issued = 4 * (depth + (steps + depth - 1) / depth * depth);  // K tiles that the waves load
+        const double tiles = g.kt + c.ahead * (issued - g.kt);
+        // 128 columns of INT4: 6% less than their fragments
+        const double load = rounds * tiles * (mr * c.a + (w4 ? 0.5 : 1.0) * nr * c.b) * (nr == 8 ? 0.94 : 1.0);
+        const double chain = std::max(0.0, (double)steps / depth - 1) * c.step;
+        const double us = c.launch + c.fill * std::min(1.0, share) + rounds * (c.round + c.frag * mr * nr) +
+                          std::sqrt(load * load + mem * mem + chain * chain);
         if (us >= best.us) continue;
         const KernelId id8[] = {K_GEMM_DIRECT16, K_GEMM_DIRECT32, K_GEMM_DIRECT64, K_GEMM_DIRECT64};
         const KernelId id4[] = {K_GEMM_W4_DIRECT16, K_GEMM_W4_DIRECT32, K_GEMM_W4_DIRECT64, K_GEMM_W4_DIRECT128};
@@ -360,23 +373,45 @@ DirectPlan plan_direct(const nh_context* ctx, int M, int N, int kt, bool w4) {
     return best;
 }
 
-// What W4A8 takes through the expanded form: a pass that reads the INT4 tiles
-// and writes int8 ones (4096 -> 16384: 17.6 us, 5.7 TB/s), then the int8 product.
-double w4_expanded_us(const nh_context* ctx, size_t m, size_t n, size_t k) {
-    const int kt = (int)tiled_k_tiles(k);
-    const double expand = 2.0 + (double)n * kt * 96 / 5.7e6;
-    double tiled;
-    tiled_gemm_cfg(ctx, (int)m, (int)n, kt, &tiled);
-    return expand + std::min(tiled, plan_direct(ctx, (int)m, (int)n, kt, false).us);
+// The int8 GEMM on tiled A: the fastest of all by those models.
+struct GemmPlan {
+    int tile;           // of kTiledCfgs, -1 for none
+    bool persistent;    // 256 x 224
+    DirectPlan direct;  // taken when neither
+    double us;
+};
+
+GemmPlan plan_gemm(const nh_context* ctx, const GemmSize& g, bool persistent_ok) {
+    GemmPlan p{-1, false, plan_direct(ctx, g, false), 0};
+    p.us = p.direct.us;
+    for (int at = 0; at < 4; ++at) {
+        const GemmCfg& c = kTiledCfgs[at];
+        if (c.lds > ctx->max_shared_per_block) continue;
+        const double us = tile_us(ctx, kTileTime[at], c.bm, c.bn, g);
+        if (us < p.us) p.tile = at, p.us = us;
+    }
+    if (persistent_ok) {
+        const double us = tile_us(ctx, kP224Time, 256, 224, g);
+        if (us < p.us) p.tile = -1, p.persistent = true, p.us = us;
+    }
+    return p;
+}
+
+// What W4A8 takes through the expanded form, without the rows' quantization: a
+// pass that reads the INT4 tiles and writes int8 ones, then the int8 product
+// (up to 16 rows the GEMV's; `fused`: one row, quantized there).  Fitted to 800
+// shapes of 1..2048 rows that were timed all ways (profiles/w4a8_choice.csv).
+double w4_expanded_us(const nh_context* ctx, const GemmSize& g, bool fused) {
+    const double expand = 2.05 + g.weights * 1.5 / 3.6;
+    if ((size_t)g.M <= kTiledActRows) return expand + 4.33 + 0.033 * g.kt + g.weights / 5.6 - (fused ? 1.5 : 0.0);
+    return expand + 1.17 * plan_gemm(ctx, g, g.M % 4 == 0 && g.N % 4 == 0 && g.kt % 2 == 0).us;
 }
 
 nh_status launch_gemm_direct(nh_context* ctx, const DirectPlan& p, const GemmW8A8Args& g, int w4_zp, float w4_scale,
                              nh_stream stream, nh_error* err) {
     GemmDirectArgs d{g, p.groups, w4_zp, w4_scale, 0};
     d.g.tiles_n = (g.N + 16 * p.nr - 1) / (16 * p.nr);
-    // partial fragments of 4 waves, row and column scales, bias, INT4 row sums
-    const size_t lds = 4 * 16 * 1024 + 3 * 128 * 4 + 4 * 128 * 4;
-    return launch(ctx, p.id, p.grid, 256u, lds, stream, d, err);
+    return launch(ctx, p.id, p.grid, 256u, kDirectLds, stream, d, err);
 }
 
 // G3 launch.  a_tiled: xq holds A in the weights' tiled layout (written by
@@ -398,33 +433,31 @@ nh_status launch_gemm(nh_context* ctx, const int8_t* xq, const float* sx, const 
     a.relu2 = relu2;
     a.kt = (int)tiled_k_tiles(K);
     a.ldo = N;
-    if (a_tiled && use_persistent_224(ctx, xq, sx, sw, bias, M, N, a.kt, out, out_dtype)) {
-        a.tiles_m = (M + 255) / 256;
-        a.tiles_n = (N + 223) / 224;
-        const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
-        const unsigned grid = (unsigned)std::min<int64_t>(tiles, ctx->cu_count);
-        return launch(ctx, K_GEMM_P224, grid, 512u, kP224Lds, stream, a, err);
-    }
-    // Tile choice.  Tiled A: by time (tiled_gemm_cfg, plan_direct).  Row-major
-    // A: 256x128 unless that leaves most CUs idle, then 128x128.
+    // Tile choice.  Tiled A: by time (plan_gemm).  Row-major A: 256x128 unless
+    // that leaves most CUs idle, then 128x128.
     const GemmCfg big = a_tiled ? kTiledCfgs[0] : GemmCfg{K_GEMM_W8A8, 256, 128, 1024, gemm_lds_bytes(256, 128, 3)};
     const GemmCfg small = a_tiled ? kTiledCfgs[1] : GemmCfg{K_GEMM_W8A8_128, 128, 128, 256, gemm_lds_bytes(128, 128, 3)};
     auto tiles = [&](const GemmCfg& c) { return gemm_tiles(c, M, N); };
     const GemmCfg* cfg = nullptr;
     if (a_tiled) {
-        double us;
-        const int at = tiled_gemm_cfg(ctx, M, N, a.kt, &us);
-        if (at >= 0) cfg = &kTiledCfgs[at];
-        // the register-direct kernel where it is faster: few or ragged tiles, long K
-        const DirectPlan p = plan_direct(ctx, M, N, a.kt, false);
-        if (p.us < us) return launch_gemm_direct(ctx, p, a, 0, 0.0f, stream, err);
+        const GemmPlan p = plan_gemm(ctx, gemm_size(M, N, a.kt, out_dtype),
+                                     persistent_224_ok(ctx, xq, sx, sw, bias, M, N, a.kt, out, out_dtype));
+        if (p.persistent) {
+            a.tiles_m = (M + 255) / 256;
+            a.tiles_n = (N + 223) / 224;
+            const int64_t n_tiles = (int64_t)a.tiles_m * a.tiles_n;
+            const unsigned grid = (unsigned)std::min<int64_t>(n_tiles, ctx->cu_count);
+            return launch(ctx, K_GEMM_P224, grid, 512u, kP224Lds, stream, a, err);
+        }
+        if (p.us >= kNoPlan) return set_error(err, NH_UNSUPPORTED, "LDS too small for the GEMM tiles");
+        if (p.tile < 0) return launch_gemm_direct(ctx, p.direct, a, 0, 0.0f, stream, err);
+        cfg = &kTiledCfgs[p.tile];
     } else if (tiles(big) >= ctx->cu_count / 4 && big.lds <= ctx->max_shared_per_block) {
         cfg = &big;
     } else if (small.lds <= ctx->max_shared_per_block) {
         cfg = &small;
     }
     if (!cfg) {
-        if (a_tiled) return set_error(err, NH_UNSUPPORTED, "LDS too small for the GEMM tiles");
         // LDS too small for the MFMA tiles: 16-row GEMV passes (still exact)
         for (int m0 = 0; m0 < M; m0 += 16) {
             const int mm = std::min(16, M - m0);
@@ -611,8 +644,9 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
         void* lin = (char*)sw + align256(n * sizeof(float));
         const size_t lin_bytes = workspace_bytes - (size_t)((char*)lin - (char*)workspace);
         // up to a few hundred rows: the register-direct GEMM on the INT4 tiles themselves
-        const DirectPlan p = plan_direct(ctx, (int)m, (int)n, (int)tiled_k_tiles(k), true);
-        if (p.us < w4_expanded_us(ctx, m, n, k))
+        const GemmSize g = gemm_size((int)m, (int)n, (int)tiled_k_tiles(k), out_dtype);
+        const DirectPlan p = plan_direct(ctx, g, true);
+        if (p.us < w4_expanded_us(ctx, g, long_row_ok(ctx, x, x_dtype, m, n, k, out, out_dtype, nullptr, nullptr)))
             return linear_w4a8_direct(ctx, p, x, x_dtype, w4_tiled, scale, zero_point, bias, m, n, k, out, out_dtype,
                                       workspace, nonfinite, stream, err);
         ExpandInt4Args e{w4_tiled, w8, sw, (int64_t)(tiled_int4_bytes(n, k) / 8), (int64_t)n, scale,
