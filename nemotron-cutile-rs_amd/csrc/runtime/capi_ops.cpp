@@ -181,13 +181,15 @@ nh_status launch_quantize(nh_context* ctx, const void* x, nh_dtype dtype, size_t
                      ((uintptr_t)q % (16 / esz)) == 0 && aligned16(q_act);
     QuantizeRowsArgs a{x, q, scales, row_status, q_act, (int64_t)rows, (int64_t)cols, dtype, vec ? 1 : 0,
                        act_p > 0 ? act_p : (int)rows, gather_div, gather, nonfinite, nonfinite_stage, 0};
-    // the GEMM's A tiles for many rows of up to 512 chunks: 8 rows per
-    // workgroup, whole 128-byte lines per store (M = 2048 linear layer,
-    // 4096 -> 4096: 45.6-45.8 us against 46.1-46.7 with the wave kernel).
-    // Fewer rows leave CUs idle that way, and a workgroup per row is faster:
-    // 77 x 4096 bf16 with its product 15.8 against 17.7 us, 800 rows 19.3
-    // against 20.6; half-length rows only below 512 (800 x 1024 f32 11.0 / 10.4).
-    const size_t tile_rows = (row_bytes > 256 * 16 ? 4 : 2) * (size_t)ctx->cu_count;
+    // the GEMM's A tiles for rows of up to 512 chunks: 8 rows per workgroup,
+    // whole 128-byte lines per store (M = 2048 linear layer, 4096 -> 4096:
+    // 45.6-45.8 us against 46.1-46.7 with the wave kernel).  A few rows of more
+    // than 1 KiB leave CUs idle that way, and a workgroup per row is faster
+    // (profiles/quantizer_choice.csv, in calls with a 256-column product, tiles /
+    // row: 288 x 64 f32 5.8 us / 6.2, 300 x 3072 bf16 0.6 more, 800 x 2048 f32
+    // 13.9 / 15.1; 1298 x 3856 bf16, 31 KiB of codes per workgroup, 21.8 / 20.6).
+    const size_t cus = (size_t)ctx->cu_count;
+    const size_t tile_rows = row_bytes <= 1024 ? 0 : row_bytes <= 2048 ? cus : cols <= 2560 ? 2 * cus : 4 * cus;
     if (vec && q_act && act_p == 16 && !gather && rows >= tile_rows && row_bytes <= 512 * 16) {
         const size_t lds = 8 * 64 * tiled_k_tiles(cols);
         return launch(ctx, K_QUANTIZE_TILES, (unsigned)((rows + 7) / 8), 512, lds, stream, a, err);
@@ -200,9 +202,10 @@ nh_status launch_quantize(nh_context* ctx, const void* x, nh_dtype dtype, size_t
         return launch(ctx, K_QUANTIZE_ROWS_WAVE, (unsigned)((rows + 3) / 4), 256, 0, stream, a, err);
     // a few rows longer than a 256-thread workgroup holds in registers
     // (1024 chunks; 2816 in the form below): 1024 threads per row, one round
-    // trip to memory (500 x 21504 f32 with its product 69.7 against 72.6 us,
-    // 1000 rows 83.5 / 86.7, 2048 rows 115.8 / 115.2)
-    if (vec && row_bytes > 1024 * 16 && rows <= (row_bytes > 2816 * 16 ? 4 : 1) * (size_t)ctx->cu_count)
+    // trip to memory; up to four rows per CU of more than 4608 chunks (500 x
+    // 21504 f32 with its product 69.7 against 72.6 us, 1000 rows 83.5 / 86.7; but
+    // 716 x 11776 f32 45.2 / 41.8, 899 x 15760 60.5 / 59.0)
+    if (vec && row_bytes > 1024 * 16 && rows <= (row_bytes > 4608 * 16 ? 4 : 1) * cus)
         return launch(ctx, K_QUANTIZE_ROWS_LONG, (unsigned)rows, 1024, 0, stream, a, err);
     // many rows of 1025..2816 chunks: the whole row in a 256-thread workgroup's
     // registers, read once (2048 x 21504 bf16: 3 us less)

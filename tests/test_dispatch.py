@@ -98,3 +98,15 @@ def test_w4a8_choice_is_near_the_best(rec):
         excess.append(next(times[k] for k in took if k in times) / min(times.values()))
     assert len(excess) >= 700
     assert sum(excess) / len(excess) < 1.015 and max(excess) < 1.34
+
+
+# The row quantizer of a GEMM's A tiles, against the times of a call with each (its 256-column product included).
+def test_quantizer_choice_is_near_the_best(rec):
+    excess = []
+    for r in choice_table("quantizer_choice.csv"):
+        # the forms that the dispatch has for the shape: a wave per row is for gathered rows, 11 chunks per thread past 1024
+        times = {k: float(v) for k, v in r.items() if k.startswith("quantize") and v and k != "quantize_rows_wave"}
+        took = rec.linear(int(r["m"]), 256, int(r["k"]), NH.F32 if r["x"] == "f32" else NH.BF16)[0]
+        excess.append(times[took] / min(times.values()))
+    assert len(excess) == 700
+    assert sum(1 for e in excess if e > 1.03) <= 25 and sum(excess) / len(excess) < 1.004
