@@ -890,15 +890,17 @@ nh_status linear_w8a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const in
         int8_t* tiles = (int8_t*)workspace;
         float* sx = sx_out ? sx_out : (float*)((char*)workspace + align256(act_tiles_bytes(m, k)));
         // The quantizer's workgroups hand the rows to the GEMV's inside one
-        // launch where that saves more than its wait costs: long rows, and
-        // every workgroup on a CU of its own (8 x 6144 -> 2048 9.9 us against
-        // 10.7 in two launches, 8 x 7680 -> 512 9.0 / 11.4; but 8 x 5120 -> 4096,
-        // 264 workgroups, 12.8 / 10.7, 5 x 2688 -> 4096 11.4 / 8.9, 12 x 688 -> 20115
-        // 23.2 / 9.3), or so much weight per workgroup that a few on shared CUs
-        // do not matter (8 x 8192 -> 4096 13.3 / 13.6, -> 6144 17.2 / 17.8).
+        // launch where that saves more than its wait costs.  Long rows with every
+        // workgroup on a CU of its own (8 x 6144 -> 2048 9.8 us against 10.4 in
+        // two launches, 8 x 7680 -> 355 8.9 / 10.7; but 5 x 2688 -> 4096 11.4 / 8.9);
+        // or, for up to 8 rows on up to 1.5 CUs' worth of workgroups, so many
+        // weights (126 K tiles per CU, 33 MB) that the rows are through before the
+        // first slab is: 8 x 8192 -> 4096 13.4 / 13.8, 7168 -> 5120 16.0 / 16.3, 8192
+        // -> 5120 17.1 / 17.8, 7680 -> 6144 17.5 / 17.8; but 7680 -> 4096 13.6 / 13.2,
+        // 5120 -> 4096 12.8 / 10.4, 5 x 6144 -> 6144 15.5 / 14.9.
         const size_t tiles_n = (n + 15) / 16, cu = (size_t)ctx->cu_count, ktiles = (size_t)tiled_k_tiles(k);
         const bool handoff = (ktiles >= 64 && tiles_n + m <= cu) ||
-                             (ktiles >= 128 && tiles_n <= cu * 3 / 2 && m <= 8);
+                             (ktiles >= 108 && tiles_n * ktiles >= 126 * cu && 2 * tiles_n <= 3 * cu && m <= 8);
         if (handoff && x_dtype == NH_BF16 && aligned16(x) && k <= 8192 && ((uintptr_t)xq_out & 7u) == 0) {
             LinearHandoffArgs h{};
             h.q = QuantizeRowsArgs{x, xq_out, sx, nullptr, tiles, (int64_t)m, (int64_t)k, x_dtype, 1, (int)m, 1,

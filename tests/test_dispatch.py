@@ -110,3 +110,14 @@ def test_quantizer_choice_is_near_the_best(rec):
         excess.append(times[took] / min(times.values()))
     assert len(excess) == 700
     assert sum(1 for e in excess if e > 1.03) <= 25 and sum(excess) / len(excess) < 1.004
+
+
+# The handoff launch, both clauses of its rule at their edges: the first K of 64 K tiles and the last of 63, the last columns
+# whose workgroups all have a CU beside the rows'; the weights per CU, the row count and the columns of the second.
+@pytest.mark.parametrize("m,n,k,handoff", [(8, 512, 4048, True), (8, 512, 4032, False), (5, 1000, 4080, True), (12, 4200, 688, False),
+                                           (16, 3840, 6160, True), (16, 3841, 6160, False), (8, 4096, 8192, True),
+                                           (9, 4096, 8192, False), (8, 4096, 8064, True), (8, 4096, 7680, False),
+                                           (8, 5120, 6912, True), (8, 5120, 6848, False), (8, 6144, 6912, True),
+                                           (8, 6144, 6144, False), (8, 6145, 8192, False)])
+def test_handoff_rule(rec, m, n, k, handoff):
+    assert rec.linear(m, n, k) == (["linear_handoff"] if handoff else ["quantize_rows_i8", "gemv_w8a8_xt"])
