@@ -123,6 +123,11 @@ extern "C" __global__ __launch_bounds__(256) void nh_gemm_f32_kernel(GemmF32Args
 // 25.0 -> 19.4, 100 x 4096 x 60 34.4 -> 24.0, 2048 x 4096 x 128 (four rounds, the
 // MFMA pipes busy) 84.2 -> 82.0.  Chunks of 128 in 108 KiB were as fast on one
 // round and 93 us on four.
+// K of one or two chunks (SHORT) has two buffers and two chunks of loads, none
+// ahead: with the third buffer's LDS two workgroups fit a CU and not four, and
+// the loads past the end cost as much as the product.  1210 x 8 x 360 8.1 -> 5.9
+// us, 546 x 107 x 101 4.6 -> 3.7, 2048 x 128 x 128 6.3 -> 5.2 (4.6 with one role
+// per wave and 16-byte rhs loads, which one round of few workgroups loses by).
 //
 // Loads go through buffer resources over the whole operands (wave-uniform;
 // the launch keeps both below 2^31 bytes), positions past the matrix sent out
@@ -138,7 +143,7 @@ constexpr int kF32APair = 320;                  // bytes of a step pair of 4 row
 constexpr int kF32AGroup = kF32Pairs * kF32APair;
 constexpr int kF32ABytes = 4 * kF32AGroup;
 constexpr int kF32Buffer = kF32ABytes + kF32Pairs * 1024;  // A of the 4 row groups, then B
-static_assert(3 * kF32Buffer == kGemmF32MfmaLds, "the host's LDS size");
+static_assert(kF32Buffer == kGemmF32MfmaBuffer, "the host's LDS size");
 
 typedef double nh_v2d __attribute__((ext_vector_type(2)));
 
@@ -220,28 +225,30 @@ struct StageB {
     }
 };
 
-template <class Stage>
+template <bool SHORT, class Stage>
 __device__ __forceinline__ void gemm_f32_stage(const Stage& s, int8_t* lds, int nc) {
-    uint32_t v[kF32Ahead][Stage::kRegs];
+    constexpr int AHEAD = SHORT ? 2 : kF32Ahead;
+    uint32_t v[AHEAD][Stage::kRegs];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < kF32Ahead; ++u) {  // (chunks past the last: zeros)
+    for (int u = 0; u < AHEAD; ++u) {  // (chunks past the last: zeros)
         s.fetch(u, v[u]);
         __builtin_amdgcn_sched_barrier(0);
     }
     int buf = 0;
-    for (int c = 0; c < nc; c += kF32Ahead) {
+    for (int c = 0; c < nc; c += AHEAD) {
 #pragma unroll
-        for (int u = 0; u < kF32Ahead; ++u) {
+        for (int u = 0; u < AHEAD; ++u) {
             if (c + u >= nc) break;  // uniform
             s.store(lds + buf * kF32Buffer, v[u]);
-            s.fetch(c + u + kF32Ahead, v[u]);
+            if constexpr (!SHORT) s.fetch(c + u + AHEAD, v[u]);
             lds_publish();  // barrier c + u
             buf = buf == 2 ? 0 : buf + 1;
         }
     }
 }
 
+template <bool SHORT>
 __device__ __forceinline__ void gemm_f32_chain(const GemmF32Args& a, const int8_t* lds, int64_t m0, int64_t n0, int nc) {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -264,7 +271,7 @@ __device__ __forceinline__ void gemm_f32_chain(const GemmF32Args& a, const int8_
     for (int p = 0; p < AHEAD; ++p) read(0, p);
     int buf = 0;
     for (int c = 0; c < nc; ++c) {
-        const int next = buf == 2 ? 0 : buf + 1;
+        const int next = SHORT ? buf ^ 1 : buf == 2 ? 0 : buf + 1;
 #pragma unroll
         for (int p = 0; p < kF32Pairs; ++p) {
             if (p == kF32Pairs / 2 && c + 1 < nc) lds_barrier();  // chunk c + 1
@@ -283,36 +290,38 @@ __device__ __forceinline__ void gemm_f32_chain(const GemmF32Args& a, const int8_
     if (gm < a.M && gn < a.N) a.out[gm * a.N + gn] = a.bias ? (float)acc + a.bias[gn] : (float)acc;
 }
 
-template <bool BF16, bool VEC>
+template <bool BF16, bool VEC, bool SHORT>
 __device__ __forceinline__ void gemm_f32_mfma(const GemmF32Args& a, int8_t* lds) {
     const int64_t tiles_n = (a.N + 15) / 16;
     const int64_t m0 = (int64_t)(blockIdx.x / tiles_n) * 16, n0 = (int64_t)(blockIdx.x % tiles_n) * 16;
     const int nc = (int)((a.K + kF32Chunk - 1) / kF32Chunk);
     if (threadIdx.x < 256)
-        gemm_f32_chain(a, lds, m0, n0, nc);
+        gemm_f32_chain<SHORT>(a, lds, m0, n0, nc);
     else if (threadIdx.x < 384)
-        gemm_f32_stage(StageA<BF16, VEC>(a, threadIdx.x - 256, m0, n0), lds, nc);
+        gemm_f32_stage<SHORT>(StageA<BF16, VEC>(a, threadIdx.x - 256, m0, n0), lds, nc);
     else
-        gemm_f32_stage(StageB(a, threadIdx.x - 384, m0, n0), lds, nc);
+        gemm_f32_stage<SHORT>(StageB(a, threadIdx.x - 384, m0, n0), lds, nc);
 }
 
 }  // namespace
 
-extern "C" __global__ __launch_bounds__(512) void nh_gemm_f32_mfma_kernel(GemmF32Args a) {
-    extern __shared__ __align__(1024) int8_t smem[];
-    gemm_f32_mfma<false, true>(a, smem);
-}
-
-extern "C" __global__ __launch_bounds__(512) void nh_gemm_f32_mfma_bf16_kernel(GemmF32Args a) {
-    extern __shared__ __align__(1024) int8_t smem[];
-    gemm_f32_mfma<true, true>(a, smem);
-}
-
-// Any alignment and K: one load per value.
-extern "C" __global__ __launch_bounds__(512) void nh_gemm_f32_mfma_any_kernel(GemmF32Args a) {
-    extern __shared__ __align__(1024) int8_t smem[];
-    if (a.lhs_bf16)
-        gemm_f32_mfma<true, false>(a, smem);
-    else
-        gemm_f32_mfma<false, false>(a, smem);
-}
+// ANY: any alignment and K, one load per value.  SHORT: K <= 128.
+#define NH_F32_MFMA_KERNEL(name, BF16, SHORT)                                      \
+    extern "C" __global__ __launch_bounds__(512) void name(GemmF32Args a) {        \
+        extern __shared__ __align__(1024) int8_t smem[];                           \
+        gemm_f32_mfma<BF16, true, SHORT>(a, smem);                                 \
+    }
+#define NH_F32_MFMA_ANY_KERNEL(name, SHORT)                                        \
+    extern "C" __global__ __launch_bounds__(512) void name(GemmF32Args a) {        \
+        extern __shared__ __align__(1024) int8_t smem[];                           \
+        if (a.lhs_bf16)                                                            \
+            gemm_f32_mfma<true, false, SHORT>(a, smem);                            \
+        else                                                                       \
+            gemm_f32_mfma<false, false, SHORT>(a, smem);                           \
+    }
+NH_F32_MFMA_KERNEL(nh_gemm_f32_mfma_kernel, false, false)
+NH_F32_MFMA_KERNEL(nh_gemm_f32_mfma_bf16_kernel, true, false)
+NH_F32_MFMA_ANY_KERNEL(nh_gemm_f32_mfma_any_kernel, false)
+NH_F32_MFMA_KERNEL(nh_gemm_f32_mfma_short_kernel, false, true)
+NH_F32_MFMA_KERNEL(nh_gemm_f32_mfma_short_bf16_kernel, true, true)
+NH_F32_MFMA_ANY_KERNEL(nh_gemm_f32_mfma_short_any_kernel, true)

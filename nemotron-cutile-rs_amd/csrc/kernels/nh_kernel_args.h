@@ -244,8 +244,10 @@ struct GemmDirectArgs {
     int32_t pad_;
 };
 
-// Dynamic LDS of the f64 matrix-core GEMM (gemm_f32.hip): three chunks of 64 k.
-constexpr int kGemmF32MfmaLds = 3 * (4 * 8 * 320 + 8 * 1024);
+// Dynamic LDS of the f64 matrix-core GEMM (gemm_f32.hip): three chunks of 64 k,
+// two for K of up to kGemmF32Short.
+constexpr int kGemmF32MfmaBuffer = 4 * 8 * 320 + 8 * 1024;
+constexpr int kGemmF32Short = 128;
 
 // R1: sigmoid top-k routing, one wave per token.
 struct RouteArgs {

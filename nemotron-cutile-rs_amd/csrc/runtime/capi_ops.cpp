@@ -785,8 +785,13 @@ static nh_status launch_gemm_f32(nh_context* ctx, const GemmF32Args& a, nh_strea
         return launch(ctx, K_GEMM_F32, (unsigned)((a.N + 63) / 64), 256, 0, stream, a, err,
                       (unsigned)((a.M + 63) / 64));
     const bool vec = aligned16(a.lhs) && a.K % (a.lhs_bf16 ? 8 : 4) == 0;
-    const KernelId id = !vec ? K_GEMM_F32_MFMA_ANY : a.lhs_bf16 ? K_GEMM_F32_MFMA_BF16 : K_GEMM_F32_MFMA;
-    return launch(ctx, id, (unsigned)(((a.M + 15) / 16) * ((a.N + 15) / 16)), 512, kGemmF32MfmaLds, stream, a, err);
+    const bool brief = a.K <= kGemmF32Short;
+    const KernelId id = !vec         ? brief ? K_GEMM_F32_MFMA_SHORT_ANY : K_GEMM_F32_MFMA_ANY
+                        : a.lhs_bf16 ? brief ? K_GEMM_F32_MFMA_SHORT_BF16 : K_GEMM_F32_MFMA_BF16
+                        : brief      ? K_GEMM_F32_MFMA_SHORT
+                                     : K_GEMM_F32_MFMA;
+    return launch(ctx, id, (unsigned)(((a.M + 15) / 16) * ((a.N + 15) / 16)), 512, (brief ? 2 : 3) * kGemmF32MfmaBuffer,
+                  stream, a, err);
 }
 
 nh_status nh_gemm_f32(nh_context* ctx, const float* lhs, size_t lhs_len, const float* rhs, size_t rhs_len, size_t m,

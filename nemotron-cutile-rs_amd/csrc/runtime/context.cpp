@@ -75,6 +75,9 @@ const char* const kKernelSymbols[K_COUNT] = {  // in KernelId order
     "nh_linear_decode_stream_w4_any_m8_kernel",   // K_LINEAR_DECODE_STREAM_W4_ANY_M8
     "nh_linear_decode_stream_w4_any_m16_kernel",  // K_LINEAR_DECODE_STREAM_W4_ANY_M16
     "nh_linear_decode_stream_w4_long_m8_kernel",  // K_LINEAR_DECODE_STREAM_W4_LONG_M8
+    "nh_gemm_f32_mfma_short_kernel",       // K_GEMM_F32_MFMA_SHORT
+    "nh_gemm_f32_mfma_short_bf16_kernel",  // K_GEMM_F32_MFMA_SHORT_BF16
+    "nh_gemm_f32_mfma_short_any_kernel",   // K_GEMM_F32_MFMA_SHORT_ANY
 };
 
 void clear_error(nh_error* err) {

@@ -78,6 +78,9 @@ enum KernelId : int {
     K_LINEAR_DECODE_STREAM_W4_ANY_M8,   // M <= 8, K <= 4096 of any multiple of 16, INT4 weights
     K_LINEAR_DECODE_STREAM_W4_ANY_M16,  // M <= 16
     K_LINEAR_DECODE_STREAM_W4_LONG_M8,  // M <= 8, K <= 8192
+    K_GEMM_F32_MFMA_SHORT,       // the f64 matrix-core GEMMs at K <= 128
+    K_GEMM_F32_MFMA_SHORT_BF16,
+    K_GEMM_F32_MFMA_SHORT_ANY,
     K_COUNT
 };
 

@@ -121,3 +121,12 @@ def test_quantizer_choice_is_near_the_best(rec):
                                            (8, 6144, 6144, False), (8, 6145, 8192, False)])
 def test_handoff_rule(rec, m, n, k, handoff):
     assert rec.linear(m, n, k) == (["linear_handoff"] if handoff else ["quantize_rows_i8", "gemv_w8a8_xt"])
+
+
+# The f64 matrix-core GEMM's two-chunk form up to K = 128, by alignment and K.
+@pytest.mark.parametrize("k,shift,kernel", [(128, 0, "short"), (132, 0, ""), (127, 0, "short_any"), (129, 0, "any"),
+                                            (64, 4, "short_any"), (4, 0, "short")])
+def test_gemm_f32_short_k(rec, k, shift, kernel):
+    m, n, X = 300, 60, 1 << 40
+    assert rec.kernels("nh_gemm_f32", X + shift, m * k, 2 << 40, k * n, m, k, n, 3 << 40, m * n, None) == [
+        "gemm_f32_mfma" + ("_" + kernel if kernel else "")]

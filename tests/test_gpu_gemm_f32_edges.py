@@ -17,7 +17,7 @@ def ctx():
     c.close()
 
 
-@pytest.mark.parametrize("k", [2, 8, 60, 64, 68, 127, 192, 256, 384, 388, 448, 453, 776])
+@pytest.mark.parametrize("k", [1, 2, 8, 60, 64, 65, 68, 127, 128, 129, 132, 192, 256, 384, 388, 448, 453, 776])
 @pytest.mark.parametrize("m,n", [(1, 16), (4, 17), (5, 1), (16, 60), (35, 130)])
 def test_gemm_f32_chunk_edges(ctx, m, n, k):
     print(f"gemm_f32 m={m} k={k} n={n}", flush=True)
