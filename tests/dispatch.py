@@ -44,3 +44,8 @@ class Recorder:
         ws = NH.lib().nh_linear_w4a8_workspace_size(m, n, k)
         return self.kernels("nh_linear_w4a8", x, x_dtype, W, 0.01, 8, None, m, n, k, out, NH.BF16, WS if workspace else None,
                             ws if workspace else 0, None, None)
+
+    def mlp(self, m, hidden, inter, x_dtype=NH.BF16, out_dtype=NH.BF16):
+        ws = NH.lib().nh_mlp_w8a8_workspace_size(m, hidden, inter)
+        return self.kernels("nh_mlp_w8a8", X, x_dtype, W, S, BIAS, W2, S2, BIAS, m, hidden, inter, OUT, out_dtype, WS, ws, None,
+                            None)

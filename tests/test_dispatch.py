@@ -1,6 +1,7 @@
 """Which kernels the entry points launch, and the rules behind that (no GPU: dispatch.py)."""
 import csv
 import os
+import re
 
 import pytest
 
@@ -130,3 +131,39 @@ def test_gemm_f32_short_k(rec, k, shift, kernel):
     m, n, X = 300, 60, 1 << 40
     assert rec.kernels("nh_gemm_f32", X + shift, m * k, 2 << 40, k * n, m, k, n, 3 << 40, m * n, None) == [
         "gemm_f32_mfma" + ("_" + kernel if kernel else "")]
+
+
+# Every linear kernel of the library is reached by a shape that the GPU tests check bit for bit: a dispatch that moves on
+# must not leave one behind without a test.
+def test_gpu_tests_reach_every_linear_kernel(rec):
+    import test_gpu_direct_gemm as direct
+    import test_gpu_parity as parity
+    import test_gpu_random_shapes as drawn
+    import test_gpu_w4_decode_any as w4any
+
+    def shapes(fn):
+        return next(m.args[1] for m in fn.pytestmark if m.name == "parametrize" and m.args[0].startswith("m,"))
+
+    reached = set()
+    for m, n, k, kernels in direct.SHAPES + direct.RAGGED:
+        reached.update(kernels)
+    for m, n, k, _, f32, offset, _ in shapes(direct.test_direct_w4a8_bit_exact):
+        reached.update(rec.w4a8(m, n, k, NH.F32 if f32 else NH.BF16, x=(1 << 40) + offset))
+    for m, n, k, _, dtype in shapes(parity.test_linear_w4a8_bit_exact):
+        reached.update(rec.w4a8(m, n, k, NH.F32 if dtype == "f32" else NH.BF16))
+    for m, n, k, _ in shapes(w4any.test_w4a8_decode_any_k_bit_exact):
+        reached.update(rec.w4a8(m, n, k))
+    for fn in (parity.test_linear_decode_unit_bit_exact, parity.test_linear_small_m_shapes_bit_exact, parity.test_linear_handoff_bit_exact):
+        for s in shapes(fn):
+            f32 = fn is parity.test_linear_small_m_shapes_bit_exact and s[3] == "f32"
+            reached.update(rec.linear(s[0], s[1], s[2], NH.F32 if f32 else NH.BF16))
+    for m, hidden, inter, dtype in shapes(parity.test_mlp_bit_exact):
+        reached.update(rec.mlp(m, hidden, inter, NH.F32 if dtype == "f32" else NH.BF16))
+    for i in range(40):
+        m, n, k, dtype, out_bf16, _, _ = drawn.draw_linear(i)
+        reached.update(rec.linear(m, n, k, NH.F32 if dtype == "f32" else NH.BF16, NH.BF16 if out_bf16 else NH.F32))
+    for m, n, k in shapes(parity.test_gemm_w8a8_bit_exact):
+        reached.update(rec.kernels("nh_gemm_w8a8", 1 << 40, 2 << 40, 3 << 40, 4 << 40, None, m, n, k, 5 << 40, NH.BF16, None))
+    source = os.path.join(os.path.dirname(NH.__file__), "csrc", "runtime", "context.cpp")
+    every = set(re.findall(r'"nh_((?:linear|gemm_w|expand)\w*)_kernel"', open(source).read()))
+    assert len(every) > 30 and every - reached == set()

@@ -19,6 +19,7 @@ import pytest
 
 import nemotron_hip as NH
 import oracle_ctypes as O
+from dispatch import Recorder
 from exact_int import linear_w8a8_exact, moe_forward_exact, moe_grouped_exact
 from tiling import tile_16x64, tile_experts
 
@@ -338,10 +339,12 @@ def test_linear_decode_unit_bit_exact(ctx, m, n, k):
                                          # (most waves past kt), K = 6144 on the 8-tile form, 17 rounds
                                          (8, 21512, 4096, "bf16"), (8, 100, 4096, "bf16"), (5, 4000, 512, "bf16"),
                                          (8, 3000, 6144, "bf16"), (6, 65544, 512, "bf16"),
+                                         # the wide unit on whole rounds of two N tiles per workgroup
+                                         (8, 8190, 7168, "bf16"), (3, 8186, 8192, "bf16"),
                                          # the persistent 256 x 224 GEMM with a bias and f32 out
                                          (1000, 14236, 384, "bf16"), (1024, 14336, 256, "f32"),
-                                         # batched decode past 16 rows: 64 x 64 tiles (M = 24, 64),
-                                         # 64 x 128 (M = 128), 128 x 128 (M = 256), ragged N and K
+                                         # batched decode past 16 rows: the register-direct GEMM (M = 24,
+                                         # 64), 64 x 64 tiles (M = 128), 128 x 128 (M = 256), ragged N and K
                                          (24, 16384, 4096, "bf16"), (64, 5000, 1040, "bf16"),
                                          (128, 16390, 512, "bf16"), (256, 16384, 2048, "f32")])
 def test_linear_small_m_shapes_bit_exact(ctx, m, n, k, dtype):
@@ -412,6 +415,15 @@ def test_linear_decode_stack_attention_shapes(ctx, n, k, out_dtype, with_bias):
         assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
 
 
+def launched(call, *args, **kwargs):
+    """The kernels that a call launches (dispatch.Recorder's method of that name)."""
+    rec = Recorder()
+    try:
+        return getattr(rec, call)(*args, **kwargs)
+    finally:
+        rec.close()
+
+
 # ---- the in-launch handoff (quantizer + tiled-A GEMV as one launch, M <= 16) ------
 def handoff_status(ctx):
     timeouts, busy = ctypes.c_uint32(0), ctypes.c_uint32(0)
@@ -419,17 +431,21 @@ def handoff_status(ctx):
     return timeouts.value, busy.value
 
 
-@pytest.mark.parametrize("m,n,k,out_dtype,with_bias", [(5, 100, 16, "f32", True), (9, 1000, 80, "bf16", False),
-                                                       (13, 4096, 528, "f32", False), (16, 4100, 8192, "bf16", True),
-                                                       (11, 16, 4112, "bf16", True), (8, 4096, 8192, "f32", True),
-                                                       (6, 2000, 4160, "bf16", False), (16, 300, 6144, "f32", True)])
-def test_linear_handoff_bit_exact(ctx, m, n, k, out_dtype, with_bias):
+@pytest.mark.parametrize("m,n,k,out_dtype,with_bias,launches", [(5, 100, 16, "f32", True, 2), (9, 1000, 80, "bf16", False, 2),
+                                                                (13, 4096, 528, "f32", False, 2), (16, 4100, 8192, "bf16", True, 2),
+                                                                (11, 16, 4112, "bf16", True, 1), (8, 4096, 8192, "f32", True, 1),
+                                                                (6, 2000, 4160, "bf16", False, 1), (16, 300, 6144, "f32", True, 1),
+                                                                (5, 1, 4048, "bf16", True, 1), (16, 3840, 8176, "f32", False, 1)])
+def test_linear_handoff_bit_exact(ctx, m, n, k, out_dtype, with_bias, launches):
     """5..16 bf16 rows that no fused decode unit takes (K % 512 != 0, K past
-    4096, or 9..16 rows at K past 4096): the quantizer's workgroups hand the
-    rows to the GEMV's workgroups inside one launch.  Codes, scales and
-    outputs bit-exact against Q2 and linear.rs:325-339's order; the context's
-    handoff slots all back at zero, no wait out of polls."""
+    4096, or 9..16 rows at K past 4096): with few columns and long rows the
+    quantizer's workgroups hand the rows to the GEMV's workgroups inside one
+    launch, otherwise the two are launches.  Codes, scales and outputs
+    bit-exact against Q2 and linear.rs:325-339's order; the context's handoff
+    slots all back at zero, no wait out of polls."""
     note(f"linear_w8a8 handoff m={m} n={n} k={k} out={out_dtype} bias={with_bias}")
+    took = launched("linear", m, n, k)
+    assert len(took) == launches and (took == ["linear_handoff"]) == (launches == 1)
     _, wq, sw = quantized_weights(n, k, seed=11)
     bias = O.normal_f32(13, n, 0.0, 0.1) if with_bias else None
     x = activations_bf16(m, k, seed=80 + m)
@@ -460,8 +476,9 @@ def test_linear_handoff_slots_wrap_and_graph_replays(ctx):
     result; then three calls captured in a HIP graph, replayed four times with
     eager calls and synchronizations between the replays, every replay
     checked."""
-    m, n, k = 8, 512, 1040
+    m, n, k = 8, 512, 4176
     note(f"linear_w8a8 handoff ring m={m} n={n} k={k}")
+    assert launched("linear", m, n, k) == ["linear_handoff"]
     _, wq, sw = quantized_weights(n, k, seed=12)
     dw, ds = ctx.upload(tile_16x64(wq)), ctx.upload(sw)
     ws_bytes = NH.lib().nh_linear_w8a8_workspace_size(m, k)
@@ -646,11 +663,14 @@ def test_gemv_w8a32_within_tolerance(ctx, m, n, k):
                                             (5, 1000, 512, 4, "bf16"), (8, 16384, 4096, 8, "bf16"),
                                             (6, 100, 2048, 15, "bf16"), (4, 21520, 1024, 0, "bf16"),
                                             (12, 16384, 4096, 1, "bf16"), (9, 6000, 512, 15, "bf16"),
-                                            # the expanded form: f32 rows, K past the fused unit's 8192,
-                                            # prefill-sized M on the GEMM (M and N tails)
+                                            # f32 rows, K past the fused unit's 8192, prefill-sized M (M and
+                                            # N tails): the register-direct GEMM on the INT4 tiles
                                             (3, 1000, 2048, 6, "f32"), (1, 600, 16384, 5, "bf16"),
                                             (17, 300, 1024, 11, "bf16"), (300, 2050, 1024, 8, "bf16"),
-                                            (129, 520, 4096, 2, "f32")])
+                                            (129, 520, 4096, 2, "f32"),
+                                            # and the weights expanded to int8 tiles: few columns of short
+                                            # rows, a prefill, one long row on few columns
+                                            (80, 100, 32, 6, "bf16"), (1500, 2050, 1024, 8, "bf16"), (1, 136, 15312, 5, "bf16")])
 def test_linear_w4a8_bit_exact(ctx, m, n, k, zp, dtype):
     """nh_linear_w4a8 against the layer's definition: or_linear_w4a8 for bf16
     rows; for f32 rows the oracle's parts (quantize_rows_f32, then the W8A8
@@ -702,8 +722,9 @@ def test_linear_w4a8_bit_exact(ctx, m, n, k, zp, dtype):
                                    # M and N (a half-valid last weight tile)
                                    (512, 8192, 64), (1000, 2000, 192), (777, 8200, 1040),
                                    # a sparse last round of 256 x 128 tiles: whole rounds, then the
-                                   # remaining columns as 128 x 128 tiles (also at 777 x 8200)
-                                   (1100, 9000, 128),
+                                   # remaining columns as 128 x 128 tiles (row-major A: also at 777 x
+                                   # 8200 and 1100 x 9000, which run on one tile with tiled A)
+                                   (1100, 9000, 128), (1225, 14755, 144),
                                    # the persistent 256 x 224 kernel (tiled A; also 2048 x 21504): one tile
                                    # per CU, and ragged last tiles in M and N with several tiles per CU
                                    (1024, 14336, 256), (1000, 14236, 384), (2000, 21484, 128)])
@@ -1273,11 +1294,14 @@ def take_nonfinite(ctx, word):
 @pytest.mark.parametrize("m,n,k,dtype", [(1, 4096, 4096, "bf16"),    # fused one-row unit
                                          (3, 4096, 8192, "bf16"),    # fused 4-row unit, one N tile per workgroup
                                          (6, 16384, 4096, "bf16"),   # fused streaming unit
-                                         (8, 4096, 8192, "bf16"),    # streaming unit, 8 K tiles per wave
-                                         (12, 1024, 4096, "bf16"),   # quantizer into activation tiles + GEMV
+                                         (8, 4096, 8192, "bf16"),    # the handoff launch
+                                         (12, 1024, 4096, "bf16"),   # streaming unit, 9..16 rows
+                                         (12, 1024, 1040, "bf16"),   # quantizer into activation tiles + GEMV
                                          (2, 1024, 4096, "f32"),     # f32 rows: the row quantizer
                                          (40, 512, 1024, "bf16"),    # quantizer into A tiles + GEMM
-                                         (41, 512, 1024, "f32"),     # the same, f32 rows, a partial 8-row group
+                                         (41, 512, 1024, "f32"),     # the same, f32 rows
+                                         (40, 512, 512, "bf16"),     # 8 rows per workgroup into A tiles
+                                         (41, 512, 256, "f32"),      # the same, f32 rows, a partial 8-row group
                                          (300, 256, 21504, "bf16"),  # long rows: a workgroup per row, re-read tail
                                          (20, 256, 21504, "f32")])   # long rows: 1024 threads per row
 def test_linear_nonfinite_input_reported(ctx, m, n, k, dtype):
@@ -1316,15 +1340,21 @@ def test_linear_nonfinite_input_reported(ctx, m, n, k, dtype):
     assert np.array_equal(word.numpy(), np.zeros(1, dtype=np.uint64))
 
 
-@pytest.mark.parametrize("m,n,k,bad", [(8, 1024, 8192, [(5, 7)]),            # groups of 4 rows: row 5 is group 2
-                                       (8, 1024, 8192, [(6, 3), (2, 100)]),  # the earlier group's index wins
-                                       (6, 1024, 4096, [(4, 9)])])          # the streaming unit (one launch)
-def test_linear_w4a8_nonfinite_input_reported(ctx, m, n, k, bad):
+@pytest.mark.parametrize("m,n,k,bad,launches", [(8, 1024, 8192, [(5, 7)], 1),
+                                                (8, 1024, 8192, [(6, 3), (2, 100)], 1),
+                                                (6, 1024, 4096, [(4, 9)], 1),                # the streaming unit
+                                                (12, 1024, 8192, [(9, 7)], 2),               # groups of 8 and 4 rows: row 9 is group 2
+                                                (13, 1024, 8192, [(12, 7), (11, 3)], 2),     # 8 and 5
+                                                (16, 1024, 8192, [(13, 3), (2, 100)], 2),    # the earlier group's index wins
+                                                (6, 262160, 16, [(5, 7)], 2),                # groups of 4 (more columns than the streaming
+                                                (6, 262160, 16, [(4, 0), (1, 15)], 2)])      # unit's runs hold): row 5 is group 2
+def test_linear_w4a8_nonfinite_input_reported(ctx, m, n, k, bad, launches):
     """nh_linear_w4a8 reports a non-finite activation at its index in the
-    whole input, also where it runs the rows in groups of 4 launches
-    (K = 8192): a NaN in row 5 is reported as 5 K + c, not as its index inside
-    the second group."""
+    whole input, also where it runs the rows in groups of 8 or 4, a launch
+    each: a NaN in row 9 is reported as 9 K + c, not as its index inside the
+    second group."""
     note(f"linear_w4a8 nonfinite m={m} n={n} k={k} bad={bad}")
+    assert len(launched("w4a8", m, n, k)) == launches
     zp, scale = 8, 0.01
     packed = np.random.default_rng(m).integers(0, 256, size=(k * n + 1) // 2, dtype=np.uint8)
     xf = O.normal_f32(70 + m, m * k).reshape(m, k)

@@ -4,7 +4,7 @@ checked against the oracle bit-exactly (the bar of test_gpu_parity.py).
 The fixed-shape tests pin each kernel at the shapes it was written for; these
 draws cross the dispatch boundaries in combinations nobody picked: rows across
 1..16 (the one-tile, wide and streaming decode units, the two-launch GEMV),
-17..513 (the GEMM on 64 x 128, 128 x 128 and 256 x 128 tiles), K on both sides
+17..513 (the register-direct GEMM and the LDS-tiled ones), K on both sides
 of 512-multiples, 4096 and 8192, ragged N from one tile to several rounds of
 CUs, bf16 and f32 rows, bf16 and f32 outputs, with and without bias; MoE
 layers from 2 to 160 experts, top-1..8, with and without renormalization and
