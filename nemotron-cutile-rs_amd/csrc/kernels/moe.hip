@@ -788,34 +788,22 @@ __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds
             //    two-deep pipeline of 4 K tiles per lane, with this wave's
             //    first two weight chunks issued behind the first two blocks
             const __amdgpu_buffer_rsrc_t hr = make_rsrc(a.ah, (uint32_t)a.a_rows * (uint32_t)K * 4u);
-            // the rows' maxima over the parts that wrote them (non-negative
-            // floats order like their bits): both of two; of more, lane group
-            // g takes parts g, g + 4, ..., eight per round trip, and the groups
-            // meet (two per round trip in every group: 3% of a one-token
-            // layer's time, 29 parts)
-            auto part_max = [&](int rb, int p) -> uint32_t {
-                const int row = p0 + rb * 16 + r16;
-                return rb < nrb && row < seg1 && p < a.ah_parts ? a.ahmax[(int64_t)row * a.ah_parts + p] : 0u;
-            };
+            // the rows' maxima over the parts that wrote them, two parts per
+            // round trip (non-negative floats order like their bits)
             uint32_t hm[4] = {0, 0, 0, 0};
             __builtin_amdgcn_sched_barrier(0);
-            const bool spread = a.ah_parts > 2;  // uniform
-            for (int p = spread ? g : 0; p < a.ah_parts; p += spread ? 8 : 2) {
+            for (int p = 0; p < a.ah_parts; p += 2) {
                 uint32_t h0[4], h1[4];
 #pragma unroll
                 for (int rb = 0; rb < 4; ++rb) {
-                    h0[rb] = part_max(rb, p);
-                    h1[rb] = part_max(rb, p + (spread ? 4 : 1));
+                    const int row = p0 + rb * 16 + r16;
+                    const bool ok = rb < nrb && row < seg1;
+                    const uint32_t* at = a.ahmax + (int64_t)row * a.ah_parts + p;
+                    h0[rb] = ok ? at[0] : 0u;
+                    h1[rb] = ok && p + 1 < a.ah_parts ? at[1] : 0u;
                 }
 #pragma unroll
                 for (int rb = 0; rb < 4; ++rb) hm[rb] = max(hm[rb], max(h0[rb], h1[rb]));
-            }
-            if (spread) {
-#pragma unroll
-                for (int rb = 0; rb < 4; ++rb) {
-                    hm[rb] = max(hm[rb], (uint32_t)__shfl_xor((int)hm[rb], 16, kWave));
-                    hm[rb] = max(hm[rb], (uint32_t)__shfl_xor((int)hm[rb], 32, kWave));
-                }
             }
             v4i hv[2][4][4];
             // the lane's 16 values of a K tile: 64 contiguous bytes in either order
