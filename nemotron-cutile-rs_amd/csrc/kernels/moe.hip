@@ -581,65 +581,36 @@ __device__ __forceinline__ void expert_stream(const ExpertGemmArgs& a, v4i (&b0)
 // consecutive workgroups: with one workgroup slot per expert, some engines got
 // two rounds of work and others none (16 tokens over 128 experts in 3 parts
 // each: 82 us per projection against 60 in 2 parts).
+// Four steps of 64 experts have their reads in flight at once: one step after
+// another, the 16 of 1024 experts made a layer up to 1.4 times as long as
+// without the search.  Counting by the whole workgroup through LDS from 193
+// experts on, over 420 layers of random sizes: 0.2-0.4% longer at up to 128
+// experts (that search not even run), 1.1-1.5 at 256 to 1024.
 __device__ __forceinline__ int nth_active_expert(const int32_t* offsets, int E, int n, int lane, int& seg0, int& seg1) {
-    for (int base = 0; base < E; base += 64) {
-        const int e = min(base + lane, E - 1);
-        const int lo = offsets[e], hi = base + lane < E ? offsets[e + 1] : lo;
-        const uint64_t live = __ballot(hi > lo);
-        const int c = __popcll(live);
-        if (n < c) {
-            const uint64_t below = live & ((1ull << lane) - 1ull);
-            const uint64_t hit = __ballot(((live >> lane) & 1) != 0 && __popcll(below) == n);
-            const int l = __ffsll((unsigned long long)hit) - 1;
-            seg0 = __builtin_amdgcn_readlane(lo, l);
-            seg1 = __builtin_amdgcn_readlane(hi, l);
-            return base + l;
+    constexpr int kSteps = 4;
+    for (int base = 0; base < E; base += 64 * kSteps) {
+        int lo[kSteps], hi[kSteps];
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {  // past the experts: empty
+            lo[s] = offsets[min(base + 64 * s + lane, E)];
+            hi[s] = offsets[min(base + 64 * s + lane + 1, E)];
         }
-        n -= c;
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            const uint64_t live = __ballot(hi[s] > lo[s]);
+            const int c = __popcll(live);
+            if (n < c) {
+                const uint64_t below = live & ((1ull << lane) - 1ull);
+                const uint64_t hit = __ballot(((live >> lane) & 1) != 0 && __popcll(below) == n);
+                const int l = __ffsll((unsigned long long)hit) - 1;
+                seg0 = __builtin_amdgcn_readlane(lo[s], l);
+                seg1 = __builtin_amdgcn_readlane(hi[s], l);
+                return base + 64 * s + l;
+            }
+            n -= c;
+        }
     }
     return -1;
-}
-
-// The same by the whole workgroup, for more experts than the wave walks in three
-// steps (a step is a dependent read of the offsets: 16 of them at 1024 experts
-// made the MoE layer up to 1.4 times as long as without the search): thread t
-// counts the experts t L .. t L + L - 1, L = ceil(E / threads), all reads in
-// flight at once.  sh: 16 words of LDS, free again on return.
-__device__ __forceinline__ int nth_active_expert_wide(const int32_t* offsets, int E, int n, int* sh, int& seg0,
-                                                      int& seg1) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, T = blockDim.x;
-    const int L = (E + T - 1) / T, e0 = min(tid * L, E), e1 = min(e0 + L, E);
-    int count = 0;
-#pragma unroll 4
-    for (int e = e0; e < e1; ++e) count += offsets[e + 1] > offsets[e];
-    int incl = count;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const int v = __shfl_up(incl, off, kWave);
-        if (lane >= off) incl += v;
-    }
-    if (lane == 63) sh[wave] = incl;
-    if (tid == 0) sh[8] = -1;
-    __syncthreads();
-    int first = incl - count;
-    for (int w = 0; w < wave; ++w) first += sh[w];
-    if (n >= first && n < first + count) {
-        int at = first;
-        for (int e = e0; e < e1; ++e) {
-            const int lo = offsets[e], hi = offsets[e + 1];
-            if (hi > lo && at++ == n) {
-                sh[8] = e;
-                sh[9] = lo;
-                sh[10] = hi;
-            }
-        }
-    }
-    __syncthreads();
-    const int e = __builtin_amdgcn_readfirstlane(sh[8]);
-    seg0 = __builtin_amdgcn_readfirstlane(sh[9]);
-    seg1 = __builtin_amdgcn_readfirstlane(sh[10]);
-    __syncthreads();
-    return e;
 }
 
 // The three forms of the expert-block kernel:
@@ -664,10 +635,7 @@ __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds
     const int part = blockIdx.x;
     int e = blockIdx.y, seg0, seg1;
     if (a.compact) {
-        if (a.experts <= 192)
-            e = nth_active_expert(a.offsets, a.experts, e, lane, seg0, seg1);
-        else
-            e = nth_active_expert_wide(a.offsets, a.experts, e, (int*)lds, seg0, seg1);
+        e = nth_active_expert(a.offsets, a.experts, e, lane, seg0, seg1);
         if (e < 0) return;  // fewer experts have routes
     } else {
         seg0 = a.offsets[e];
