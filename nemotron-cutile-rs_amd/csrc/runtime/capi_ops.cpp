@@ -33,8 +33,9 @@ int gemv_waves(int kt) { return std::max(1, std::min(8, (kt + 15) / 16)); }
 // The linear entry point's M ranges: the fused decode unit (quantizer inside
 // the GEMV, one launch) for up to 4 bf16 rows (K <= 8192) and for 3..16 bf16
 // rows (K <= 4096, K % 512 == 0, the streaming form), and for one f32 or longer
-// row (long_row_ok); other bf16 rows up to 16 with K = 4096..8192 and few
-// columns as the handoff launch (quantizer workgroups feeding the tiled-A
+// row that no output overlaps (long_row_ok); other bf16 rows up to 16 with K =
+// 4048..8192 on a grid that the CUs take at once, or of weights enough to hide
+// the rows, as the handoff launch (quantizer workgroups feeding the tiled-A
 // GEMV's workgroups inside one launch); otherwise quantization into
 // activation tiles + the tiled-A GEMV up to 16 rows, and the MFMA GEMMs beyond.
 constexpr size_t kTiledActRows = 16;
@@ -326,9 +327,9 @@ struct DirectPlan {
 // Its model: a launch, more with more CUs taking part; per round (or partly,
 // INT4, per CU's share of one: two workgroups of a CU overlap there) an
 // epilogue per fragment, and per K tile the fragments through the CU's load
-// path (`a` and `b` us per KiB: 80 KiB per us), also, at `ahead` of the cost,
-// for the loads past the end that a wave's `depth` K tiles in flight round up
-// to; beside that the memory traffic and a wave's chain of dependent
+// path (`a` us per KiB of activations, `b` of weights: 93 and 69 KiB per us), also, at
+// `ahead` of the cost, for the loads past the end that a wave's `depth` K tiles
+// in flight round up to; beside that the memory traffic and a wave's chain of dependent
 // steps.  Against the LDS tiles, both measured at M x N x K: 17 x 2688 x 2688
 // 5.5 / 11.8 us, 77 x 6144 x 4096 11.5 / 15.8, 400 x 2688 x 4096 15.5 / 20.9, 64 x
 // 16384 x 1024 7.8 / 6.8, 512 x 16384 x 4096 49.2 / 36.2.
@@ -635,8 +636,9 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
     if ((st = check_dtype(x_dtype, err)) || (st = check_dtype(out_dtype, err))) return st;
     if (((uintptr_t)w4_tiled & 7u) != 0) return set_error(err, NH_UNSUPPORTED, "w4_tiled must be 8-byte aligned");
     if (x_dtype != NH_BF16 || !nh_supports_linear_w4a8(m, n, k) || !aligned16(x)) {
-        // any other shape or f32 rows: the weights expanded into int8 tiles of
-        // code - zp (the layer's definition) and the W8A8 linear path on them
+        // any other shape, f32 or unaligned rows: the register-direct GEMM on the
+        // INT4 tiles, or the weights expanded into int8 tiles of code - zp (the
+        // layer's definition) and the W8A8 linear path on them, by their times
         if ((st = check_w8a8_shape(m, n, k, err))) return st;
         const size_t need = nh_linear_w4a8_workspace_size(m, n, k);
         if (!workspace || workspace_bytes < need) return mismatch(err, "workspace", need, workspace_bytes);
@@ -646,7 +648,6 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
         float* sw = (float*)(w8 + align256((size_t)tiled_bytes(n, k)));
         void* lin = (char*)sw + align256(n * sizeof(float));
         const size_t lin_bytes = workspace_bytes - (size_t)((char*)lin - (char*)workspace);
-        // up to a few hundred rows: the register-direct GEMM on the INT4 tiles themselves
         const GemmSize g = gemm_size((int)m, (int)n, (int)tiled_k_tiles(k), out_dtype);
         const DirectPlan p = plan_direct(ctx, g, true);
         if (p.us < w4_expanded_us(ctx, g, long_row_ok(ctx, x, x_dtype, m, n, k, out, out_dtype, nullptr, nullptr)))
@@ -1186,20 +1187,18 @@ static nh_status launch_expert_gemm(nh_context* ctx, KernelId id, ExpertGemmArgs
     e.streams = kExpertWaves;
     e.tiles_per_wg = tiles_per_wg;
     e.row_blocks = row_blocks;
-    // Packed onto the experts with routes (a search of 0.2-0.9 us per launch)
-    // where their workgroups then fit one round of CUs and would not in natural
-    // order: more slots than CUs, and so many of them live that some CUs would
-    // get two (half the CUs' worth, or one of 4 slots per CU and up); or, past
-    // one round, where three of four experts have no route.  Natural order /
-    // packed, us: 128 experts of 1168 x 688 with 16 routes 48.7 / 36.5 per
-    // layer, 64 of 1312 x 2560 with 14 71.1 / 53.8, 253 of 272 x 2192 with 112
-    // 20.1 / 13.3; but 16 of 1024 x 512 with 12 31.1 / 31.5, 197 of 240 x 368
-    // with 216 (262 workgroups packed) 9.9 / 11.6, 1024 of 192 x 1408 with 620
-    // 62.1 / 70.2.
+    // Packed onto the experts with routes (a search of 0.2-0.6 us per launch)
+    // where slots in natural order would give some CUs two live workgroups
+    // and others none: as many slots as CUs and more, a tenth of the experts
+    // without routes, and the live ones 0.4 of the CUs' worth or the slots three
+    // per CU.  Natural order / packed, us per layer: 256 experts of 624 x 512 with 198
+    // routes 55.3 / 41.5, 64 of 2048 x 1024 with 128 (4 slots each) 77.3 / 74.2, 1024
+    // of 2048 x 96 with 684 168.2 / 143.2, 128 of 2688 x 1856 with 2 53.4 / 48.3; but
+    // 64 of 960 x 1024 with 153 (nine in ten) 45.2 / 46.5, 60 of 336 x 512 with 2
+    // 26.1 / 26.7.  On 800 layers of 16 to 1024 experts within 0.3% of the best
+    // of both orders on average (packed wherever a tenth has none: 0.5%).
     const double cu = ctx->cu_count, live = expected_experts(experts, routes), all = (double)parts * (double)experts;
-    const double packed = parts * live;
-    e.compact = all > cu && (packed <= cu ? 2 * packed >= cu || all > 4 * cu
-                                          : (double)experts >= 4 * live && packed <= 4 * cu);
+    e.compact = all >= cu && live < 0.9 * (double)experts && (parts * live >= 0.4 * cu || all >= 3 * cu);
     const size_t slots = e.compact ? std::min(experts, routes) : experts;
     return launch(ctx, id, (unsigned)parts, (unsigned)(64 * kExpertWaves), lds, stream, e, err, (unsigned)slots);
 }
