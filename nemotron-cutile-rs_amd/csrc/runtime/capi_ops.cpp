@@ -1197,8 +1197,12 @@ static nh_status launch_expert_gemm(nh_context* ctx, KernelId id, ExpertGemmArgs
     // 64 of 960 x 1024 with 153 (nine in ten) 45.2 / 46.5, 60 of 336 x 512 with 2
     // 26.1 / 26.7.  On 800 layers of 16 to 1024 experts within 0.3% of the best
     // of both orders on average (packed wherever a tenth has none: 0.5%).
+    // Past 1024 experts the search is long, and an empty workgroup leaves as
+    // soon: packed up to three rounds (6297 of 416 x 64 with 1979 routes 82 / 145 us a launch,
+    // 12302 of 16 x 64 with 1234 56.7 / 134; but 2457 of 16 x 3584 with 114 16.2 / 11.5).
     const double cu = ctx->cu_count, live = expected_experts(experts, routes), all = (double)parts * (double)experts;
-    e.compact = all >= cu && live < 0.9 * (double)experts && (parts * live >= 0.4 * cu || all >= 3 * cu);
+    e.compact = all >= cu && live < 0.9 * (double)experts && (parts * live >= 0.4 * cu || all >= 3 * cu) &&
+                (experts <= 1024 || parts * live <= 3 * cu);
     const size_t slots = e.compact ? std::min(experts, routes) : experts;
     return launch(ctx, id, (unsigned)parts, (unsigned)(64 * kExpertWaves), lds, stream, e, err, (unsigned)slots);
 }

@@ -62,7 +62,7 @@ def test_w4a8_decode_ignores_its_workspace(rec, m, k):
 @pytest.mark.parametrize("experts,routes,parts,slots", [(16, 12, 8, 16), (136, 1, 8, 1), (30, 1, 8, 30), (128, 126, 2, 126), (127, 126, 2, 127),
                                                         (128, 48, 4, 48), (128, 3072, 2, 128), (184, 125, 2, 125),
                                                         (512, 300, 2, 300), (1024, 48, 4, 48), (1024, 180, 2, 180),
-                                                        (1024, 1428, 2, 1024)])
+                                                        (1024, 1428, 2, 1024), (1025, 500, 2, 1025), (4000, 380, 2, 380)])
 def test_expert_slots(rec, experts, routes, parts, slots):
     (name, gx, gy), = rec.launches("nh_moe_grouped_gemm_w8a8", 1 << 40, 2 << 40, 0, 1, 3 << 40, 4 << 40, routes, routes, experts,
                                    5 << 40, 6 << 40, 512, 1024, 0, 7 << 40, None)
