@@ -195,7 +195,7 @@ nh_status nh_take_nonfinite(nh_context *ctx, uint64_t *nonfinite, nh_stream stre
  * k <= 8192 and m <= 4 (m <= 16 when k % 512 == 0 and k <= 4096) the
  * quantization is fused into the GEMV (one launch; the workspace is not
  * touched), as it is for most single rows of f32 or of k > 8192 (which still
- * ask for their workspace); some bf16 x with m <= 16 and 4096 <= k <= 8192 is
+ * ask for their workspace); some bf16 x with m <= 16 and 4032 < k <= 8192 is
  * one launch whose quantizer workgroups hand the codes to its GEMV workgroups
  * through the workspace and a counter slot of the context (kHandoffSlots = 256
  * slots taken in turn: at most 256 such launches may be in flight at once on

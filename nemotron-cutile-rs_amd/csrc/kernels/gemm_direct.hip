@@ -8,16 +8,15 @@
 // and its four waves split K: wave w takes K tiles w, w + 4, ...  Both operands
 // are stored in MFMA operand order (tiled A, tiled weights), so every fragment
 // is one contiguous 16-byte-per-lane load; the K loop has no LDS and no barrier,
-// each wave keeps D K tiles in flight and waits for exact load counts.  The four
-// partial tiles meet in LDS once, at the end (int32 sums: exact in any order).
+// each wave keeps D K tiles in flight.  The four partial tiles meet in LDS once,
+// at the end (int32 sums: exact in any order).
 //
-// What bounds it: the CU's vector-memory path returns loads in order and holds
-// about 64 KiB in flight, so a CU moves 64 KiB per round trip of its slowest
-// loads (the weights' from HBM): 57-60 KB/us measured, whatever the registers
-// could hold.  A K tile costs MR + NR KiB there (MR + NR / 2 with INT4 weights);
-// the tile shape, a function of the launch, keeps that small while filling the
-// CUs (launch_gemm_direct).  Workgroups are dealt so that the row groups of a
-// column block run side by side on one XCD, whose L2 then reads the weights once.
+// What bounds it: the CU's vector-memory path, 65.7 KiB/us over the whole launch
+// at 500 x 4096 x 21504 (256 workgroups of 336 K tiles of 12 KiB in 61.4 us).  A K
+// tile costs MR + NR KiB there (MR + NR / 2 with INT4 weights); the tile shape, a
+// function of the launch, keeps that small while filling the CUs (plan_direct).
+// Workgroups are dealt so that the row groups of a column block run side by side
+// on one XCD, whose L2 then reads the weights once.
 //
 // Measured against the LDS-tiled kernels (tiled A in, cold weights):
 // 33 x 4096 x 8192 29.7 -> 13.0 us, 77 x 6144 x 4096 15.8 -> 11.5, 256 x 2688 x

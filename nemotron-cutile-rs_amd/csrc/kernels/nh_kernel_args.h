@@ -123,8 +123,9 @@ struct LinearHandoffArgs {
     int32_t pad_;
 };
 
-// Decode unit (M <= 16, K <= 8192, K % 512 == 0): per-token quantization
-// (Q2) of bf16 rows fused in front of G1.  A workgroup owns ntw 16-row N
+// Decode units (M <= 16, K <= 8192; K % 512 == 0 in the streaming form with int8
+// weights, M = 1 of any K or f32 in the long-row form): per-token quantization
+// (Q2) of the rows fused in front of G1.  A workgroup owns ntw 16-row N
 // tiles with `waves` waves each: blockDim = 64 * waves * ntw <= 1024 and
 // waves * 1024 >= 64 * kt.
 struct LinearDecodeArgs {
@@ -302,8 +303,8 @@ struct GroupedGemmArgs {
 };
 
 // R3, the MoE layer's form: A already in slot (expert) order.  grid =
-// (wgs_per_expert, experts); workgroup (nb, e) owns expert e's N tiles
-// [nb * tiles_per_wg, +tiles_per_wg), dealt to its `streams` waves
+// (parts, experts that can have routes); workgroup (nb, e) owns the e-th expert's
+// (the e-th with routes when `compact`) N tiles [nb * tiles_per_wg, +tiles_per_wg), dealt to its `streams` waves
 // (blockDim = 64 * streams), each wave computing whole tiles.
 struct ExpertGemmArgs {
     const int8_t* aq;        // [R][K] codes in slot order
