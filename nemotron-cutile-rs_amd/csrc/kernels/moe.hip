@@ -756,22 +756,34 @@ __device__ __forceinline__ void expert_gemm(const ExpertGemmArgs& a, int8_t* lds
             //    two-deep pipeline of 4 K tiles per lane, with this wave's
             //    first two weight chunks issued behind the first two blocks
             const __amdgpu_buffer_rsrc_t hr = make_rsrc(a.ah, (uint32_t)a.a_rows * (uint32_t)K * 4u);
-            // the rows' maxima over the parts that wrote them, two parts per
-            // round trip (non-negative floats order like their bits)
+            // the rows' maxima over the parts that wrote them (non-negative
+            // floats order like their bits): both of two at once; of more, lane
+            // group g takes parts g, g + 4, ..., eight per round trip, and the
+            // groups meet.  Against two per round trip in every group, behind
+            // branches per row block, 700 layers: 1.4% less (8 experts of 4096 x
+            // 1792, 14 parts, 5.5%; 128 of 2688 x 1856, two parts, 0.5%).
             uint32_t hm[4] = {0, 0, 0, 0};
-            __builtin_amdgcn_sched_barrier(0);
-            for (int p = 0; p < a.ah_parts; p += 2) {
-                uint32_t h0[4], h1[4];
+            auto maxima = [&](int p, int q) {  // rows past the segment: the last row's
+                uint32_t h[4][2];
 #pragma unroll
                 for (int rb = 0; rb < 4; ++rb) {
-                    const int row = p0 + rb * 16 + r16;
-                    const bool ok = rb < nrb && row < seg1;
-                    const uint32_t* at = a.ahmax + (int64_t)row * a.ah_parts + p;
-                    h0[rb] = ok ? at[0] : 0u;
-                    h1[rb] = ok && p + 1 < a.ah_parts ? at[1] : 0u;
+                    const uint32_t* at = a.ahmax + (int64_t)min(p0 + rb * 16 + r16, seg1 - 1) * a.ah_parts;
+                    h[rb][0] = at[p];
+                    h[rb][1] = at[q];
                 }
 #pragma unroll
-                for (int rb = 0; rb < 4; ++rb) hm[rb] = max(hm[rb], max(h0[rb], h1[rb]));
+                for (int rb = 0; rb < 4; ++rb) hm[rb] = max(hm[rb], max(h[rb][0], h[rb][1]));
+            };
+            __builtin_amdgcn_sched_barrier(0);
+            if (a.ah_parts <= 2) {
+                maxima(0, a.ah_parts - 1);
+            } else {
+                for (int p = g; p < a.ah_parts; p += 8) maxima(p, min(p + 4, a.ah_parts - 1));
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb) {
+                    hm[rb] = max(hm[rb], (uint32_t)__shfl_xor((int)hm[rb], 16, kWave));
+                    hm[rb] = max(hm[rb], (uint32_t)__shfl_xor((int)hm[rb], 32, kWave));
+                }
             }
             v4i hv[2][4][4];
             // the lane's 16 values of a K tile: 64 contiguous bytes in either order
