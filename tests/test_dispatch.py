@@ -5,6 +5,7 @@ import re
 
 import pytest
 
+import dispatch as D
 import nemotron_hip as NH
 from dispatch import Recorder
 
@@ -89,6 +90,15 @@ def test_gemm_choice_is_near_the_best(rec, part, mean, worst):
         excess.append(times[took[0]] / min(times.values()))
     assert len(excess) >= 300
     assert sum(excess) / len(excess) < mean and max(excess) < worst
+
+
+# A column block's row groups are on one XCD, so 20 blocks of 11 groups are 33 workgroups on some XCDs of 32 CUs: two
+# rounds.  (16 blocks are one.)
+@pytest.mark.parametrize("m,n,k,kernel", [(1309, 640, 2048, "gemm_w8a8_ta_64x64"), (1429, 576, 2592, "gemm_w8a8_ta_64x64"),
+                                          (1309, 512, 2048, "gemm_w8a8_direct32")])
+def test_gemm_choice_counts_the_rounds_of_an_xcd(rec, m, n, k, kernel):
+    (name, gx, _), = rec.launches("nh_gemm_w8a8_ta", D.X, D.S, D.W, D.S2, None, m, n, k, D.OUT, NH.BF16, None)
+    assert name == kernel and gx <= D.CUS
 
 
 def test_w4a8_choice_is_near_the_best(rec):
