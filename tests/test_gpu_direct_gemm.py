@@ -36,7 +36,7 @@ T256, T128, T64128, T6464 = (["gemm_w8a8_ta_" + t] for t in ("256x128", "128x128
 # of 4; one K tile, fewer K tiles than waves, K tails; column blocks not a multiple of the 8 XCDs
 SHAPES = [(1, 16, 16, D16), (17, 1000, 1024, D16), (64, 130, 4112, D16), (65, 2688, 2688, D16), (113, 333, 4096, D16),
           (129, 1027, 4096, D16), (400, 70, 8192, D16), (22, 18, 256, D16), (37, 122, 1040, D16), (188, 124, 2064, D16),
-          (260, 2690, 1856, D32), (120, 262, 2064, D32), (17, 5044, 1040, D32), (237, 139, 2064, D32), (372, 191, 2064, D32),
+          (260, 2498, 1856, D32), (120, 262, 2064, D32), (17, 5044, 1040, D32), (237, 139, 2064, D32), (372, 191, 2064, D32),
           (37, 11008, 4096, D64), (17, 8486, 2064, D64), (20, 10395, 2064, D64), (136, 4119, 2064, D64), (153, 4277, 2064, D64)]
 # the LDS tiles with ragged edges both ways and rows of odd length, the persistent 256 x 224 kernel with few rows in its
 # tile, and the launch split in whole rounds of 256 x 128 tiles and 128 x 128 ones for the columns after them, which are
