@@ -1065,7 +1065,7 @@ extern "C" __global__ __launch_bounds__(1024) void nh_linear_decode_stream_w4_m1
     linear_decode_stream<16, 8, 4, 2, true>(a, lds);
 }
 
-// 5..16 rows of the other K on INT4 tiles: up to 4096 in one launch, past
+// 5..16 rows of the other K on INT4 tiles (and 3..4, plan_stream_w4_any): up to 4096 in one launch, past
 // that 8 rows at a time with 8 K tiles per wave (the codes of 16 would not fit
 // the LDS).  Bound by the quantization in every workgroup ahead of few rounds
 // of weights.  Against groups of 4 rows, each streaming the weights: 5 x 288 ->

@@ -117,10 +117,15 @@ bool plan_stream(const nh_context* ctx, size_t m, size_t n, size_t k, DecodePlan
     return plan_stream_grid(ctx, kid, mm, n, k, p, grid);
 }
 
-// The INT4 form of 5..16 rows for the other K (multiples of 16): up to 4096,
-// and up to 8 rows past that.
+// The INT4 form of 3..16 rows for the other K (multiples of 16): up to 4096,
+// and up to 8 rows past that.  The one-tile unit quantizes 1..4 rows in every
+// workgroup: at 3..4 it keeps short K, and the long form's narrow outputs (3
+// rows, one-tile / this: K = 272 x 4096 5.4 us / 6.5, 1040 x 4096 6.8 / 6.9, 2064 x 4096 7.6 /
+// 7.4, 4080 x 40960 26.8 / 17.5; 4640 x 8192 11.0 / 12.1, x 10000 17.4 / 14.4, x 40960 55.1 /
+// 25.8); 2 rows are the same or slower here up to 24576 columns.
 bool plan_stream_w4_any(const nh_context* ctx, size_t m, size_t n, size_t k, DecodePlan* p, unsigned* grid) {
     if (m > (k <= 4096 ? 16u : 8u) || k > 8192) return false;
+    if (m <= 2 || (m <= 4 && (k <= 4096 ? k < 1024 : n <= 32 * (size_t)ctx->cu_count))) return false;
     const KernelId kid = k > 4096 ? K_LINEAR_DECODE_STREAM_W4_LONG_M8
                          : m <= 8 ? K_LINEAR_DECODE_STREAM_W4_ANY_M8
                                   : K_LINEAR_DECODE_STREAM_W4_ANY_M16;
@@ -690,11 +695,11 @@ nh_status nh_linear_w4a8(nh_context* ctx, const void* x, nh_dtype x_dtype, const
         return launch(ctx, kid, grid, 1024u, plan.lds, stream, a, err);
     }
     // otherwise launches over groups of rows, each streaming the weights once:
-    // all of 5..16 rows of K <= 4096, 5..8 past that, and groups of up to 4 by the
-    // one-tile units.  No workspace: a call may share its buffer with others.
+    // all of up to 16 rows of K <= 4096, up to 8 past that, and small groups by the
+    // one-tile units (plan_stream_w4_any).  No workspace: a call may share its buffer with others.
     for (size_t r0 = 0, rows; r0 < m; r0 += rows) {
         rows = std::min<size_t>(k <= 4096 ? 16 : 8, m - r0);
-        const bool wide = rows > 4 && plan_stream_w4_any(ctx, rows, n, k, &plan, &grid);
+        const bool wide = plan_stream_w4_any(ctx, rows, n, k, &plan, &grid);
         if (!wide) rows = std::min<size_t>(4, rows);
         const size_t mm = rows == 1 ? 1 : rows <= 2 ? 2 : 4;
         const KernelId kid = mm == 1 ? K_LINEAR_DECODE_W4_M1 : mm == 2 ? K_LINEAR_DECODE_W4_ROW2 : K_LINEAR_DECODE_W4_ROW4;

@@ -46,6 +46,15 @@ def test_single_row_under_its_own_outputs_takes_two_launches(rec, x_dtype, k):
     assert rec.linear(1, n, k, x_dtype, sx_out=X + row) == ["linear_decode_long"]
 
 
+# W4A8 of 3..4 rows, alone or left over from a long-K group of eight: streamed where K is not short, or the output wide.
+@pytest.mark.parametrize("m,n,k,kernels", [
+    (3, 64, 1008, ["row4"]), (4, 64, 1040, ["stream_w4_any_m8"]), (2, 64, 1040, ["row2"]), (3, 8192, 4112, ["row4"]),
+    (4, 8193, 4112, ["stream_w4_long_m8"]), (2, 30000, 4112, ["row2"]), (11, 8208, 4112, ["stream_w4_long_m8"] * 2),
+    (12, 256, 8192, ["stream_w4_long_m8", "row4"]), (9, 30000, 8192, ["stream_w4_long_m8", "m1"])])
+def test_w4a8_few_rows(rec, m, n, k, kernels):
+    assert [q.replace("linear_decode_", "").replace("w4a8_", "") for q in rec.w4a8(m, n, k)] == kernels
+
+
 # W4A8 decode never writes the workspace, given or not: a buffer that calls on several streams share is not raced on.
 @pytest.mark.parametrize("m", range(1, 17))
 @pytest.mark.parametrize("k", [16, 288, 512, 1040, 4080, 4096, 4112, 5120, 8176, 8192])

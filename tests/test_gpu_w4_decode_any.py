@@ -1,4 +1,4 @@
-"""W4A8 decode of 5..16 bf16 rows whose K the 512-wide streaming unit does not take: its padded forms.  Results are exact,
+"""W4A8 decode of 3..16 bf16 rows whose K the 512-wide streaming unit does not take: its padded forms.  Results are exact,
 a non-finite value is reported at its index in the whole input, and a caller's workspace is left alone (a program may pass
 one buffer to calls on several streams: these shapes never needed it)."""
 import numpy as np
@@ -29,11 +29,14 @@ def setup(ctx, m, n, k, zp, seed):
 
 # one chunk pair, a K tile less and more one 16-group, groups of 64 chunks less and more one chunk pair, both ends of the
 # short and of the long form; one to eight and nine to sixteen rows, two launches of the long form with a remainder of one
-# row, of four and of more; one column, part of a tile, several rounds of tiles per workgroup; zero points at both ends
+# row, of four and of more; one column, part of a tile, several rounds of tiles per workgroup; zero points at both ends; three and four
+# rows on both sides of their lines, and as the remainder of eleven
 @pytest.mark.parametrize("m,n,k,zp", [(5, 1, 16, 8), (16, 40, 48, 15), (8, 100, 80, 0), (9, 517, 496, 7), (16, 256, 528, 8),
                                       (13, 4130, 1040, 3), (8, 33, 4080, 8), (16, 2048, 4080, 15), (5, 64, 4112, 8),
                                       (8, 517, 8176, 1), (8, 4100, 8192, 8), (9, 300, 8192, 15), (12, 96, 5120, 0),
-                                      (15, 130, 6160, 9), (16, 517, 8192, 6), (7, 20000, 144, 8)])
+                                      (15, 130, 6160, 9), (16, 517, 8192, 6), (7, 20000, 144, 8),
+                                      (3, 33, 1008, 8), (3, 33, 1024 + 16, 8), (4, 4130, 4080, 3), (3, 8200, 4112, 8),
+                                      (4, 8192, 4112, 15), (11, 8200, 4160, 0)])
 def test_w4a8_decode_any_k_bit_exact(ctx, m, n, k, zp):
     print(f"w4a8 decode any K m={m} n={n} k={k} zp={zp}", flush=True)
     rng, packed, x, dt = setup(ctx, m, n, k, zp, m * 131 + k)
@@ -57,7 +60,7 @@ def test_w4a8_decode_any_k_bit_exact(ctx, m, n, k, zp):
 
 
 @pytest.mark.parametrize("m,k,bad", [(16, 1040, [(15, 1039)]), (8, 6160, [(7, 6150), (7, 6159)]), (16, 8192, [(12, 3), (9, 8191)]),
-                                     (9, 8192, [(8, 5)]), (16, 4080, [(3, 4079), (11, 0)])])
+                                     (9, 8192, [(8, 5)]), (3, 1040, [(2, 1039)]), (16, 4080, [(3, 4079), (11, 0)])])
 def test_w4a8_decode_any_k_reports_the_first_nonfinite(ctx, m, k, bad):
     n = 48
     print(f"w4a8 decode any K nonfinite m={m} k={k}", flush=True)
